@@ -1,0 +1,778 @@
+"""The work that programs using this engine have it do, as timed cases.
+
+listed() names the cases, draw() gives more of the same ranges, prepare()
+makes what a program holds before the call, run() is one pass through the
+public entry points (dida_letkf.py), work() the bytes and operations a pass
+cannot do without, and exact() the same outputs in plain 64-bit torch.
+
+Kinds:
+  core       letkf_core_ / letkf_core_r4_: one local analysis, host arrays
+  batch      letkf_core_batch_ / letkf_core_batch_r4_: host arrays
+  dev        dida_letkf_core_batch_dev: device arrays
+  sweep      dida_letkf_sweep (_f32): every column of a grid
+  obsop      dida_letkf_obs_operator: H(Xb) and centring
+  cycle      what surrounds the sweep in a cycle: coupler blocks into the
+             state, the post-analysis blend, the analysis back to the coupler
+"""
+import math
+import os
+import sys
+
+import numpy as np
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "dida-thhpca-sc23_amd")
+if PKG not in sys.path:
+    sys.path.insert(0, PKG)
+import dida_letkf as dl  # noqa: E402
+
+DEV = "cuda"
+F64 = torch.float64
+FORMS = {"plain": (dl.FORM_PLAIN, dl.GRAM_FP64), "batched": (dl.FORM_BATCHED, dl.GRAM_FP64),
+         "bf16x3": (dl.FORM_BATCHED, dl.GRAM_BF16X3), "fp16x3": (dl.FORM_BATCHED, dl.GRAM_FP16X3)}
+MAX_OBS = 10000
+PTOP = 10.0          # hPa
+EARTH = float(np.float32(6371.393))
+PI32 = float(np.float32(math.pi))
+
+
+def _sweep(name, nlat, nlon, nz, k, nobs, L, form, clustered=0.0, rmin=1.0, rmax=1.0, rho=1.0,
+           rtps=0.0, f32=False, cube_n=1, overlap=0, vert=0.0, cube_nz=1):
+    c = dict(kind="sweep", nlat=nlat, nlon=nlon, nz=nz, k=k, nobs=nobs, L=L, form=form,
+             clustered=clustered, rmin=rmin, rmax=rmax, rho=rho, rtps=rtps, f32=f32,
+             cube_n=cube_n, overlap=overlap, vert=vert, cube_nz=cube_nz)
+    return dict(name=name, **c) if name else c
+
+
+def listed():
+    return [
+        # the Fortran drop-in, called once per grid point by a program that
+        # keeps its own loop: the mean local problem of the 2.5 degree workload
+        dict(name="core_one", kind="core", k=20, p=245, r4=False),
+        # the batched drop-in on host arrays, 64 members, ragged obs counts
+        dict(name="core_batch_host", kind="batch", batch=512, p=2100, k=64, r4=False),
+        # the batched core on device arrays, for a program with its own
+        # selection on the GPU
+        dict(name="core_batch_dev", kind="dev", batch=4096, p=512, k=32),
+        # the 2.5 degree, 20-member workload in the default (plain FP64) form:
+        # the smallest whole sweep, where launches count
+        _sweep("sweep_2p5deg_k20_plain", 72, 144, 8, 20, 10000, 1000.0, "plain", rho=1.1),
+        # 1 degree, 32 members, obs in clusters: local counts 0 to about 1500
+        _sweep("sweep_1deg_k32_bf16x3", 180, 360, 16, 32, 100000, 200.0, "bf16x3",
+               clustered=0.7, rho=1.1),
+        # the grid of the reference's own runs (360 x 180 x 32, 64 members) in
+        # the plain FP64 form that replaces its loop one for one
+        _sweep("sweep_1deg_k64_plain", 180, 360, 32, 64, 100000, 600.0, "plain", clustered=0.7,
+               rmin=0.1, rmax=10.0, rtps=0.8),
+        # the 0.5 degree workload of the benchmark, split BF16 contractions
+        _sweep("sweep_halfdeg_k64_bf16x3", 360, 720, 32, 64, 400000, 600.0, "bf16x3",
+               clustered=0.7, rmin=0.1, rmax=10.0, rtps=0.8),
+        # the reference's overlapping cubes at its namelist defaults (block
+        # interval 4, overlap 2), FP64 batched form
+        _sweep("sweep_1deg_k64_cubes", 180, 360, 32, 64, 100000, 600.0, "batched",
+               clustered=0.7, cube_n=4, overlap=2),
+        # vertical localisation: one analysis per column and level
+        _sweep("sweep_2p5deg_k32_vertical", 72, 144, 16, 32, 20000, 1000.0, "batched", rho=1.1,
+               vert=0.5),
+        # 128 members with the state kept in FP32, split BF16 contractions
+        _sweep("sweep_1deg_k128_f32", 180, 360, 32, 128, 125000, 600.0, "bf16x3", clustered=0.5,
+               rmin=0.5, rmax=3.0, f32=True),
+        # the observation operator on single-level records of u, v and T
+        dict(name="obs_operator", kind="obsop", nlat=180, nlon=360, nz=32, k=64, nrec=100000,
+             onz=1, onv=3, hybrid=False),
+        # coupler in, post-analysis blend, coupler out, at the reference's
+        # 100 km, 32-member configuration
+        dict(name="cycle_1deg_k32", kind="cycle", nlat=180, nlon=360, nz=32, k=32),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["core", "batch", "dev", "sweep", "sweep", "sweep", "sweep", "obsop",
+                       "cycle"])
+    if kind == "core":
+        return dict(kind="core", k=rng.randint(8, 128), p=_log(rng, 20, 4000),
+                    r4=rng.random() < 0.3)
+    if kind == "batch":
+        return dict(kind="batch", batch=_log(rng, 8, 512), p=_log(rng, 40, 2100),
+                    k=rng.randint(10, 64), r4=rng.random() < 0.3)
+    if kind == "dev":
+        k = rng.choice([rng.randint(8, 32), rng.randint(33, 64), rng.randint(65, 128)])
+        return dict(kind="dev", batch=_log(rng, 16, 8192 if k <= 64 else 2048),
+                    p=_log(rng, 16, 700), k=k)
+    nlat = _log(rng, 36, 150)
+    nlon = nlat + rng.randint(nlat // 2, nlat)
+    nz = _log(rng, 4, 32)
+    if kind == "obsop":
+        onz = rng.choice([1, 1, 2, 5])
+        return dict(kind="obsop", nlat=nlat, nlon=nlon, nz=nz, k=rng.randint(16, 128),
+                    nrec=_log(rng, 500, 100000 // onz), onz=onz, onv=rng.randint(1, 3),
+                    hybrid=rng.random() < 0.5)
+    if kind == "cycle":
+        return dict(kind="cycle", nlat=nlat, nlon=nlon, nz=nz, k=rng.randint(10, 64))
+    ncol = nlat * nlon
+    L = float(rng.choice([200, 300, 500, 600, 800, 1000]))
+    nobs = max(50, int(ncol * math.exp(rng.uniform(math.log(0.2), math.log(2.5)))))
+    cl = rng.choice([0.0, 0.5, 0.7])
+    spread = rng.random() < 0.5
+    opt = dict(clustered=cl, rmin=0.1 if spread else 1.0, rmax=10.0 if spread else 1.0,
+               rho=rng.choice([1.0, 1.05, 1.1]), rtps=rng.choice([0.0, 0.0, 0.8]))
+    shape = rng.choice(["columns", "columns", "columns", "cubes", "vertical", "large"])
+    if shape == "cubes":
+        n, o = rng.choice([(2, 0), (3, 1), (4, 2), (4, 0)])
+        return _sweep(None, nlat, nlon, nz, rng.randint(16, 64), nobs, L,
+                      rng.choice(["plain", "batched", "bf16x3"]), cube_n=n, overlap=o, **opt)
+    if shape == "vertical":
+        nlat, nlon = min(nlat, 72), min(nlon, 144)
+        return _sweep(None, nlat, nlon, min(nz, 16), rng.randint(16, 48), min(nobs, 20000), L,
+                      rng.choice(["batched", "bf16x3"]), vert=rng.choice([0.3, 0.5, 1.0]),
+                      cube_nz=rng.choice([1, 2, 4]), **opt)
+    if shape == "large":
+        nlat, nlon = min(nlat, 80), min(nlon, 160)
+        return _sweep(None, nlat, nlon, nz, rng.randint(65, 128), min(nobs, 30000), L,
+                      rng.choice(["plain", "batched", "bf16x3"]), f32=rng.random() < 0.5, **opt)
+    return _sweep(None, nlat, nlon, nz, rng.randint(10, 64), nobs, L,
+                  rng.choice(["plain", "plain", "batched", "bf16x3", "fp16x3"]), **opt)
+
+
+# ----------------------------------------------------------------------------
+# Inputs: smooth random fields (random Fourier features of a Gaussian kernel
+# on the sphere), members correlated over 500 km and over adjacent levels,
+# obs of u, v and T at random model levels.
+
+def _unit(lat, lon):
+    la, lo = torch.deg2rad(lat), torch.deg2rad(lon)
+    return torch.stack([la.cos() * lo.cos(), la.cos() * lo.sin(), la.sin()], -1)
+
+
+class _Field:
+    def __init__(self, g, nz, k, nb=320, length_km=500.0):
+        self.nz, self.k, self.nb = nz, k, nb
+        n = 1 + 3 * nz
+        self.w = torch.randn(3, nb, generator=g, device=DEV, dtype=F64) * (6371.0 / length_km)
+        self.ph = torch.rand(nb, generator=g, device=DEV, dtype=F64) * (2 * math.pi)
+        self.w0 = torch.randn(3, 24, generator=g, device=DEV, dtype=F64) * 2.0
+        self.p0 = torch.rand(24, generator=g, device=DEV, dtype=F64) * (2 * math.pi)
+        c = torch.randn(nb, n, k + 1, generator=g, device=DEV, dtype=F64)
+        for v in range(3):
+            for lev in range(1, nz):
+                r = 1 + v * nz + lev
+                c[:, r] = 0.8 * c[:, r - 1] + 0.6 * c[:, r]
+        sig = torch.tensor([1.0] + [1.5] * (2 * nz) + [1.0] * nz, device=DEV, dtype=F64)
+        c *= sig[None, :, None]
+        mean = c[:, :, :k].mean(2)
+        self.pert = (c[:, :, :k] - mean[:, :, None]).contiguous()  # (nb, n, k)
+        self.truth = (c[:, :, k] - mean).contiguous()              # truth - xbar
+        self.mean = mean
+        self.cb = torch.randn(24, n, generator=g, device=DEV, dtype=F64)
+        self.amp = torch.tensor([20.0] + [30.0] * (3 * nz), device=DEV, dtype=F64)
+        self.off = torch.tensor([1000.0] + [0.0] * (2 * nz) + [250.0] * nz, device=DEV, dtype=F64)
+
+    def phi(self, x):
+        return torch.cos(x @ self.w + self.ph) * math.sqrt(2.0 / self.nb)
+
+    def background(self, x):
+        base = torch.cos(x @ self.w0 + self.p0) * math.sqrt(2.0 / 24) @ self.cb
+        return self.off + self.amp * 0.5 * base + self.phi(x) @ self.mean
+
+
+def _grid(nlat, nlon):
+    lat = (-90.0 + (torch.arange(nlat, dtype=F64) + 0.5) * (180.0 / nlat)).float().to(DEV)
+    lon = (torch.arange(nlon, dtype=F64) * (360.0 / nlon)).float().to(DEV)
+    return lat, lon
+
+
+def _columns(lat, lon):
+    """Latitude and longitude (degrees) of every column, latitude fastest."""
+    return lat.double().repeat(lon.numel()), lon.double().repeat_interleave(lat.numel())
+
+
+def _positions(g, n, clustered):
+    z = torch.rand(n, generator=g, device=DEV, dtype=F64) * 2 - 1
+    lat = torch.rad2deg(torch.asin(z))
+    lon = torch.rand(n, generator=g, device=DEV, dtype=F64) * 360.0
+    if clustered > 0.0:
+        cz = torch.rand(6, generator=g, device=DEV, dtype=F64) * 1.6 - 0.8
+        clat, clon = torch.asin(cz), torch.rand(6, generator=g, device=DEV, dtype=F64) * (2 * math.pi)
+        c = torch.stack([clat.cos() * clon.cos(), clat.cos() * clon.sin(), clat.sin()], -1)
+        which = torch.randint(0, 6, (n,), generator=g, device=DEV)
+        x = c[which] + torch.randn(n, 3, generator=g, device=DEV, dtype=F64) * (800.0 / 6371.0)
+        x = x / x.norm(dim=1, keepdim=True)
+        inside = torch.rand(n, generator=g, device=DEV, dtype=F64) < clustered
+        lat = torch.where(inside, torch.rad2deg(torch.asin(x[:, 2].clamp(-1, 1))), lat)
+        lon = torch.where(inside, torch.rad2deg(torch.atan2(x[:, 1], x[:, 0])) % 360.0, lon)
+    return lat, lon
+
+
+def _sweep_inputs(case, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    nz, k, nobs = case["nz"], case["k"], case["nobs"]
+    n = 1 + 3 * nz
+    lat, lon = _positions(g, nobs, case["clustered"])
+    glat, glon = _grid(case["nlat"], case["nlon"])
+    f = _Field(g, nz, k)
+    cla, clo = _columns(glat, glon)
+    x = _unit(cla, clo)
+    ncol = cla.numel()
+    xb = torch.empty(ncol, n, k, dtype=torch.float32 if case["f32"] else F64, device=DEV)
+    coef = f.pert.reshape(f.nb, n * k)
+    for c0 in range(0, ncol, 32768):
+        p = f.phi(x[c0:c0 + 32768])
+        if case["f32"]:
+            xb[c0:c0 + 32768] = (p @ coef).reshape(-1, n, k).float()
+        else:
+            torch.mm(p, coef, out=xb[c0:c0 + 32768].view(-1, n * k))
+    axb = f.background(x)
+    # obs: one of u, v, T at a random level
+    row = torch.randint(1, n, (nobs,), generator=g, device=DEV)
+    order = torch.argsort(row)
+    counts = torch.bincount(row, minlength=n).cpu().tolist()
+    yb = torch.empty(nobs, k, dtype=F64, device=DEV)
+    dep = torch.empty(nobs, dtype=F64, device=DEV)
+    xo = _unit(lat, lon)
+    at = 0
+    for r in range(n):
+        if counts[r]:
+            idx = order[at:at + counts[r]]
+            p = f.phi(xo[idx])
+            yb[idx] = p @ f.pert[:, r]
+            dep[idx] = p @ f.truth[:, r]
+            at += counts[r]
+    scale = torch.exp(torch.empty(nobs, device=DEV, dtype=F64).uniform_(
+        math.log(case["rmin"]), math.log(case["rmax"]) + 1e-12, generator=g))
+    var = torch.where(row > 2 * nz, 1.0, 2.25) * scale
+    dep += torch.randn(nobs, generator=g, device=DEV, dtype=F64) * var.sqrt()
+    ph = 100.0 + 900.0 * torch.rand(nobs, generator=g, device=DEV, dtype=F64)
+    return dict(grid_lat=glat, grid_lon=glon, lat=lat, lon=lon, yb=yb, dep=dep,
+                rinv=(1.0 / var).float(), ph=ph, xb=xb, axb=axb)
+
+
+def _sigma(nz):
+    return torch.linspace(0.0, 1.0, nz + 1, dtype=F64, device=DEV)
+
+
+def _layout(nz):
+    return [0, 1, 1 + nz, 1 + 2 * nz], [1, nz, nz, nz]
+
+
+def _params(case):
+    form, gram = FORMS[case["form"]]
+    kw = dict(nanals=case["k"], nrow=1 + 3 * case["nz"], nlat=case["nlat"], nlon=case["nlon"],
+              local_dist=case["L"], inflation_factor=case["rho"], form=form, gram=gram,
+              max_obs=MAX_OBS, cube_n=case["cube_n"], overlap=case["overlap"])
+    if case["rtps"] > 0.0:
+        kw.update(rtps=1, rtps_alpha=case["rtps"])
+    if case["vert"] > 0.0:
+        kw.update(vert_dist=case["vert"], cube_nz=case["cube_nz"], gc_filter_vertical=1)
+    return dl.default_params(**kw)
+
+
+def _core_inputs(case, seed):
+    """Host arrays of local problems: Yb of smooth members at the obs, GC
+    weights of obs spread evenly over the support."""
+    rng = np.random.default_rng(seed)
+    batch, p, k = case.get("batch", 1), case["p"], case["k"]
+    nf = 48
+    f = rng.standard_normal((batch, p, nf))
+    f[..., 8:] *= 0.4
+    c = rng.standard_normal((batch, nf, k + 1)) / math.sqrt(nf / 4)
+    y = f @ c
+    hx = y[..., :k] - y[..., :k].mean(-1, keepdims=True)
+    ri = (1.0 / np.exp(rng.uniform(math.log(0.3), math.log(3.0), (batch, p)))).astype(np.float32)
+    dep = y[..., k] - y[..., :k].mean(-1) + rng.standard_normal((batch, p)) / np.sqrt(ri)
+    rl = _gc_np(2.0 * np.sqrt(rng.uniform(0.0, 0.999, (batch, p))))
+    nb = rng.integers(max(1, p // 4), p + 1, batch).astype(np.int32)
+    return nb, np.ascontiguousarray(hx), ri, dep, rl
+
+
+def _gc_np(r):
+    near = (((-0.25 * r + 0.5) * r + 0.625) * r - 5.0 / 3.0) * r * r + 1.0
+    rf = np.maximum(r, 0.5)
+    far = ((((rf / 12.0 - 0.5) * rf + 0.625) * rf + 5.0 / 3.0) * rf - 5.0) * rf + 4.0 \
+        - 2.0 / 3.0 / rf
+    return np.maximum(np.where(r <= 1.0, near, far), 0.0)
+
+
+def _dev_inputs(case, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    batch, p, k, nf = case["batch"], case["p"], case["k"], 48
+
+    def randn(*s):
+        return torch.randn(*s, generator=g, device=DEV, dtype=F64)
+
+    def rand(*s):
+        return torch.rand(*s, generator=g, device=DEV, dtype=F64)
+
+    f = randn(batch, p, nf)
+    f[..., 8:] *= 0.4
+    y = torch.bmm(f, randn(batch, nf, k + 1) / math.sqrt(nf / 4))
+    mean = y[..., :k].mean(-1)
+    hx = (y[..., :k] - mean[..., None]).contiguous()
+    ri = torch.exp(math.log(0.3) + math.log(10.0) * rand(batch, p)).float()
+    dep = y[..., k] - mean + randn(batch, p) / ri.double().sqrt()
+    r = 2.0 * (0.999 * rand(batch, p)).sqrt()
+    rl = torch.from_numpy(_gc_np(r.cpu().numpy())).to(DEV)
+    nb = torch.randint(max(1, p // 4), p + 1, (batch,), generator=g, device=DEV,
+                       dtype=torch.int32)
+    return nb, hx, ri, dep.contiguous(), rl
+
+
+def _vcoord(case):
+    nz = case["nz"]
+    s = _sigma(nz)
+    if case.get("hybrid"):
+        return dict(type=1, c1=(s * (1 - s)).contiguous(), c2=(s * s).contiguous(), ptop=PTOP,
+                    p0=1000.0)
+    return dict(type=0, c1=s, ptop=PTOP)
+
+
+def _obsop_inputs(case, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    nz, k, nrec = case["nz"], case["k"], case["nrec"]
+    n = 1 + 3 * nz
+    lat, lon = _positions(g, nrec, 0.5)
+    glat, glon = _grid(case["nlat"], case["nlon"])
+    f = _Field(g, nz, k, nb=128)
+    x = _unit(*_columns(glat, glon))
+    xb = torch.empty(x.shape[0], n, k, dtype=F64, device=DEV)
+    coef = f.pert.reshape(f.nb, n * k)
+    for c0 in range(0, x.shape[0], 32768):
+        torch.mm(f.phi(x[c0:c0 + 32768]), coef, out=xb[c0:c0 + 32768].view(-1, n * k))
+    ph = 30.0 + 1000.0 * torch.rand(nrec, case["onz"], generator=g, device=DEV, dtype=F64)
+    yo = 250.0 + 10.0 * torch.randn(nrec, case["onz"], case["onv"], generator=g, device=DEV,
+                                    dtype=F64)
+    return dict(grid_lat=glat, grid_lon=glon, xb=xb, axb=f.background(x), lat=lat, lon=lon,
+                ph=ph.sort(1).values.contiguous(), yo=yo, vid=list(range(1, 1 + case["onv"])))
+
+
+def _cycle_inputs(case, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    nz, k, nlat, nlon = case["nz"], case["k"], case["nlat"], case["nlon"]
+    n = 1 + 3 * nz
+    atm, atm_a = [], []
+    for v, lev in enumerate([1, nz, nz, nz]):
+        atm.append(torch.randn(lev, nlat, nlon, k, generator=g, device=DEV, dtype=F64))
+        atm_a.append(250.0 + 30.0 * torch.randn(lev, nlat, nlon, generator=g, device=DEV,
+                                                dtype=F64))
+    xa = 0.7 * torch.randn(nlon * nlat, n, k, generator=g, device=DEV, dtype=F64)
+    xa -= xa.mean(2, keepdim=True)
+    axa = 250.0 + 30.0 * torch.randn(nlon * nlat, n, generator=g, device=DEV, dtype=F64)
+    return atm, atm_a, xa, axa
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind in ("core", "batch"):
+        nb, hx, ri, dep, rl = _core_inputs(case, seed)
+        if case["r4"]:
+            hx, dep, rl = hx.astype(np.float32), dep.astype(np.float32), rl.astype(np.float32)
+        return dict(case=case, nb=nb, hx=hx, ri=ri, dep=dep, rl=rl)
+    if kind == "dev":
+        nb, hx, ri, dep, rl = _dev_inputs(case, seed)
+        batch, k = case["batch"], case["k"]
+        return dict(case=case, nb=nb, hx=hx, ri=ri, dep=dep, rl=rl,
+                    trans=torch.empty(batch, k, k, dtype=F64, device=DEV),
+                    wbar=torch.empty(batch, k, dtype=F64, device=DEV))
+    if kind == "sweep":
+        d = _sweep_inputs(case, seed)
+        eng = dl.Engine(_params(case), nobs_max=case["nobs"])
+        eng.set_grid(d["grid_lat"], d["grid_lon"])
+        if case["vert"] > 0.0:
+            eng.set_levels(dict(type=0, c1=_sigma(case["nz"]), ptop=PTOP), 0, *_layout(case["nz"]))
+        obs = dl.DeviceObs(d["lat"], d["lon"], d["yb"], d["dep"], d["rinv"],
+                           d["ph"] if case["vert"] > 0.0 else None)
+        return dict(case=case, eng=eng, obs=obs, xb=d["xb"], axb=d["axb"],
+                    xa=torch.empty_like(d["xb"]), axa=torch.empty_like(d["axb"]))
+    if kind == "obsop":
+        return dict(case=case, vc=_vcoord(case), **_obsop_inputs(case, seed))
+    atm, atm_a, xa, axa = _cycle_inputs(case, seed)
+    nz, k, nlat, nlon = case["nz"], case["k"], case["nlat"], case["nlon"]
+    n = 1 + 3 * nz
+
+    def new(*s):
+        return torch.zeros(*s, dtype=F64, device=DEV)
+
+    return dict(case=case, atm=atm, atm_a=atm_a, xa=xa, axa=axa, grid_lat=_grid(nlat, nlon)[0],
+                xb=new(nlon, nlat, n, k), axb=new(nlon, nlat, n), out=new(nlon, nlat, n, k),
+                sb=new(nlon * nlat, n), sa=new(nlon * nlat, n),
+                back=[torch.empty_like(t) for t in atm],
+                back_a=[torch.empty_like(t) for t in atm_a])
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "core":
+        f = dl.letkf_core_r4 if case["r4"] else dl.letkf_core
+        trans, wbar = f(state["hx"][0], state["ri"][0], state["dep"][0], state["rl"][0], 1.05)
+        return {"trans": trans, "wbar": wbar}
+    if kind == "batch":
+        f = dl.letkf_core_batch_r4 if case["r4"] else dl.letkf_core_batch
+        trans, wbar = f(state["nb"], state["hx"], state["ri"], state["dep"], state["rl"], 1.05)
+        return {"trans": trans, "wbar": wbar}
+    if kind == "dev":
+        dl.core_batch_dev(state["nb"], state["hx"], state["ri"], state["dep"], state["rl"],
+                          state["trans"], state["wbar"], 1.05)
+        return {"trans": state["trans"], "wbar": state["wbar"]}
+    if kind == "sweep":
+        state["eng"].sweep(state["obs"], state["xb"], state["axb"], state["xa"], state["axa"])
+        return {"xa": state["xa"], "axa": state["axa"]}
+    nz = case["nz"]
+    start, lev = _layout(nz)
+    if kind == "obsop":
+        lat, lon, yb, dep = dl.obs_operator(
+            state["grid_lat"], state["grid_lon"], state["xb"], state["axb"], 0, state["vc"],
+            start, lev, state["vid"], state["lat"], state["lon"], state["ph"], state["yo"])
+        return {"lat": lat, "lon": lon, "yb": yb, "dep": dep}
+    xb, axb, out = state["xb"], state["axb"], state["out"]
+    for v in range(4):
+        dl.struct_atm2endnn(1, start[v] + 1, state["atm"][v], xb)
+        dl.struct_atm2endnn_a(start[v] + 1, state["atm_a"][v], axb)
+    dl.post(case["k"], 1 + 3 * nz, case["nlat"], case["nlon"], state["grid_lat"], 85.0, 0.3, 0.7,
+            xb, axb, state["xa"], state["axa"], out, state["sb"], state["sa"])
+    axa = state["axa"].view(case["nlon"], case["nlat"], 1 + 3 * nz)
+    for v in range(4):
+        dl.struct_endnn2atm(1, start[v] + 1, out, state["back"][v])
+        dl.struct_endnn2atm_a(start[v] + 1, axa, state["back_a"][v])
+    return {"xb": xb, "axb": axb, "xa_out": out, "spread_b": state["sb"],
+            "spread_a": state["sa"], "atm": state["back"], "atm_a": state["back_a"]}
+
+
+# ----------------------------------------------------------------------------
+# What a pass cannot do without.
+
+def _transform_flops(k, nanal, nobsl_sum):
+    # symmetric Gram, b, eigensolve 9 k^3, W (symmetric) k^3, wbar
+    return k * k * nobsl_sum + 2.0 * k * nobsl_sum + nanal * (10.0 * k ** 3 + 4.0 * k * k)
+
+
+def _centres(case):
+    """Latitude and longitude of every analysis (columns, or the lower-middle
+    columns of the horizontal cubes), latitude fastest."""
+    glat, glon = _grid(case["nlat"], case["nlon"])
+    n, o = case["cube_n"], case["overlap"]
+    if n == 1:
+        return _columns(glat, glon)
+
+    def mid(size):
+        s = torch.arange(0, size, n - o)
+        return (s + (s + n - 1).clamp(max=size - 1)) // 2
+
+    return _columns(glat[mid(case["nlat"]).to(DEV)], glon[mid(case["nlon"]).to(DEV)])
+
+
+def work(case):
+    kind, k = case["kind"], case["k"]
+    if kind in ("core", "batch", "dev"):
+        batch, p = case.get("batch", 1), case["p"]
+        tot = float(p) if kind == "core" else batch * 0.625 * p
+        s = 4 if case.get("r4") else 8
+        return {"bytes": tot * (s * (k + 2) + 4) + batch * k * (k + 1) * s,
+                "flops": _transform_flops(k, batch, tot)}
+    nz, ncol = case["nz"], case["nlat"] * case["nlon"]
+    n = 1 + 3 * nz
+    if kind == "obsop":
+        ns = case["nrec"] * case["onz"] * case["onv"]
+        corners = min(4.0 * case["nrec"], float(ncol)) * k * 8
+        rows = 1 + min(2 * case["onz"], nz) * case["onv"]
+        return {"bytes": corners * rows + ns * (8 * k + 40.0), "flops": ns * k * 24.0}
+    if kind == "cycle":
+        return {"bytes": ncol * n * (k * 7 + 10) * 8.0, "flops": ncol * n * k * 10.0}
+    # local obs counts on a sample of the analyses
+    g = torch.Generator(device=DEV).manual_seed(0)
+    lat, lon = _positions(g, case["nobs"], case["clustered"])
+    cla, clo = _centres(case)
+    nsel = cla.numel()
+    at = torch.arange(0, nsel, max(1, nsel // 256), device=DEV)
+    near = math.cos(min(math.pi, 2.0 * case["L"] / EARTH))
+    dots = _unit(cla[at], clo[at]) @ _unit(lat, lon).T
+    mean_p = (dots > near).sum(1).clamp(max=MAX_OBS).double().mean().item()
+    nq = -(-nz // case["cube_nz"]) if case["vert"] > 0.0 else 1
+    part = min(1.0, 2.0 * case["vert"] / math.log(10.0)) if nq > 1 else 1.0
+    s = 4 if case["f32"] else 8
+    return {"bytes": ncol * n * (2.0 * k * s + 16.0) + case["nobs"] * (8.0 * k + 28.0),
+            "flops": _transform_flops(k, nsel * nq, nsel * nq * mean_p * part)
+            + 2.0 * k * k * n * ncol}
+
+
+# ----------------------------------------------------------------------------
+# The same outputs in plain 64-bit torch.
+
+def _analysis(y, r, d, rho):
+    """trans = W + wbar 1^T and wbar of dense local problems: y (B, p, k), r =
+    R^-1 rloc and d (B, p)."""
+    k = y.shape[-1]
+    yr = y * r[..., None]
+    c = torch.bmm(yr.transpose(1, 2).contiguous(), y)
+    b = torch.bmm(yr.transpose(1, 2).contiguous(), d[..., None])
+    lam, v = torch.linalg.eigh(0.5 * (c + c.transpose(1, 2)))
+    lam = lam + (k - 1) / rho
+    vt = v.transpose(1, 2).contiguous()
+    w = torch.bmm(v * torch.sqrt((k - 1) / lam)[:, None, :], vt)
+    wbar = torch.bmm(v, torch.bmm(vt, b) / lam[..., None])
+    return w + wbar, wbar[..., 0]
+
+
+def _gc(r):
+    c53, c23 = float(np.float32(1.666667)), float(np.float32(0.6666667))
+    near = (((-0.25 * r + 0.5) * r + 0.625) * r - c53) * r * r + 1.0
+    rf = r.clamp(min=0.5)
+    far = ((((rf / 12.0 - 0.5) * rf + 0.625) * rf + c53) * rf - 5.0) * rf + 4.0 - c23 / rf
+    return torch.where(r > 2.0, 0.0, torch.where(r > 1.0, far, near))
+
+
+def _lists(case, d, cla, clo, c0, c1):
+    """Local obs of analyses [c0, c1) in the caller's order, at most MAX_OBS
+    each: (analysis - c0, obs, weight) per kept pair."""
+    xc, xo = _unit(cla[c0:c1], clo[c0:c1]), _unit(d["lat"], d["lon"])
+    cut = math.cos(min(math.pi, 2.0 * case["L"] / EARTH * (1 + 1e-5) + 1e-6))
+    a, o = torch.nonzero(xc @ xo.T > cut, as_tuple=True)
+
+    def rad(x):
+        return x / 180.0 * PI32
+
+    x1, y1 = rad(cla[c0:c1])[a], rad(clo[c0:c1])[a]
+    x2, y2 = rad(d["lat"])[o], rad(d["lon"])[o]
+    v = (x1.cos() * x2.cos() * (y1 - y2).cos() + x1.sin() * x2.sin()).clamp(max=1.0)
+    w = _gc(EARTH * torch.acos(v) / case["L"])
+    keep = w > 0.0
+    a, o, w = a[keep], o[keep], w[keep]
+    cnt = torch.bincount(a, minlength=c1 - c0)
+    rank = torch.arange(a.numel(), device=DEV) - (cnt.cumsum(0) - cnt)[a]
+    keep = rank < MAX_OBS
+    return a[keep], o[keep], w[keep], rank[keep], cnt.clamp(max=MAX_OBS)
+
+
+def _exact_trans(case, d, scale_of=None):
+    """Yields (analysis ids, trans) over all analyses; scale_of(obs, ids)
+    scales the weights."""
+    cla, clo = _centres(case)
+    nsel, k = cla.numel(), case["k"]
+    step = max(1, (1 << 27) // max(1, case["nobs"]))
+    for c0 in range(0, nsel, step):
+        c1 = min(nsel, c0 + step)
+        a, o, w, rank, cnt = _lists(case, d, cla, clo, c0, c1)
+        order = torch.argsort(cnt)
+        sizes = cnt[order].cpu().tolist()
+        slot = torch.empty_like(order)
+        slot[order] = torch.arange(order.numel(), device=DEV)
+        sa = slot[a]
+        i = 0
+        while i < len(sizes):
+            j = i + 1
+            while j < len(sizes) and (j + 1 - i) * max(1, sizes[j]) * k <= 1 << 28:
+                j += 1
+            pmax = max(1, sizes[j - 1])
+            m = (sa >= i) & (sa < j)
+            idx = torch.zeros(j - i, pmax, dtype=torch.int64, device=DEV)
+            wt = torch.zeros(j - i, pmax, dtype=F64, device=DEV)
+            idx[sa[m] - i, rank[m]] = o[m]
+            wt[sa[m] - i, rank[m]] = w[m]
+            ids = order[i:j] + c0
+            if scale_of is None:
+                r = d["rinv"][idx].double() * wt
+                yield ids, None, _analysis(d["yb"][idx], r, d["dep"][idx], case["rho"])[0]
+            else:
+                y, dd = d["yb"][idx], d["dep"][idx]
+                for q, s in scale_of(idx, ids):
+                    r = d["rinv"][idx].double() * (wt * s)
+                    yield ids, q, _analysis(y, r, dd, case["rho"])[0]
+            i = j
+
+
+def _exact_update(case, xb, axb, trans):
+    """Xa' and xbar_a of columns: xb (B, r, k), axb (B, r), trans (B, k, k)."""
+    xa = torch.bmm(xb, trans) + axb[..., None]
+    mean = xa.mean(-1)
+    xa = xa - mean[..., None]
+    if case["rtps"] > 0.0:
+        sb, sa = xb.square().mean(-1).sqrt(), xa.square().mean(-1).sqrt()
+        fac = case["rtps"] * sb / sa + 1.0 - case["rtps"]
+        xa = xa * torch.where(sa > 0.0, fac, 1.0)[..., None]
+    return xa, mean
+
+
+def _exact_sweep(case, seed):
+    nq = -(-case["nz"] // case["cube_nz"]) if case["vert"] > 0.0 else 1
+    step = case["cube_n"] - case["overlap"]
+    nsel = -(-case["nlat"] // step) * -(-case["nlon"] // step)
+    if nsel * nq * float(case["k"]) ** 3 > 2.0e10:
+        return None  # its eigensolves alone take too long
+    d = _sweep_inputs(case, seed)
+    nz, k, nlat, nlon = case["nz"], case["k"], case["nlat"], case["nlon"]
+    xb, axb = d["xb"], d["axb"]
+    xa = torch.empty(xb.shape, dtype=F64, device=DEV)
+    axa = torch.empty_like(axb)
+    if case["vert"] > 0.0:
+        start, lev = _layout(nz)
+        s = _sigma(nz)
+        half = s[None, :] * (axb[:, :1] - PTOP) + PTOP
+        full = 0.5 * (half[:, :-1] + half[:, 1:])
+        lnp_o = torch.log(d["ph"])
+        rows, centre = [], []
+        for q in range(nq):
+            sk, ek = q * case["cube_nz"], min((q + 1) * case["cube_nz"], nz) - 1
+            centre.append((sk + ek + 2) // 2 - 1)
+            r = [start[v] + j for v in range(1, 4) for j in range(sk, ek + 1)]
+            rows.append(torch.tensor(([0] if q == nq - 1 else []) + r, device=DEV))
+
+        def scale_of(idx, ids):
+            for q in range(nq):
+                lnp_c = torch.log(full[ids, centre[q]])
+                yield q, _gc((lnp_c[:, None] - lnp_o[idx]).abs() / case["vert"])
+
+        for ids, q, t in _exact_trans(case, d, scale_of):
+            r = rows[q]
+            x, m = _exact_update(case, xb[ids][:, r].double(), axb[ids][:, r], t)
+            xa[ids[:, None], r[None, :]] = x
+            axa[ids[:, None], r[None, :]] = m
+        return {"xa": xa, "axa": axa}
+    if case["cube_n"] == 1:
+        for ids, _, t in _exact_trans(case, d):
+            for b in range(0, ids.numel(), 4096):
+                i = ids[b:b + 4096]
+                xa[i], axa[i] = _exact_update(case, xb[i].double(), axb[i], t[b:b + 4096])
+    else:
+        # every column takes the mean transform of the cubes that cover it
+        nalat, nalon = -(-nlat // step), -(-nlon // step)
+        trans = torch.empty(nalat * nalon, k, k, dtype=F64, device=DEV)
+        for ids, _, t in _exact_trans(case, d):
+            trans[ids] = t
+        for lon in range(nlon):
+            lat = torch.arange(nlat, device=DEV)
+            t = torch.zeros(nlat, k, k, dtype=F64, device=DEV)
+            cnt = torch.zeros(nlat, dtype=F64, device=DEV)
+            for ai in range(nalon):
+                if not ai * step <= lon <= ai * step + case["cube_n"] - 1:
+                    continue
+                for back in range(-(-case["cube_n"] // step)):
+                    aj = lat // step - back
+                    ok = (aj >= 0) & (lat <= aj * step + case["cube_n"] - 1)
+                    t += torch.where(ok[:, None, None], trans[aj.clamp(min=0) + nalat * ai], 0.0)
+                    cnt += ok
+            i = lat + nlat * lon
+            xa[i], axa[i] = _exact_update(case, xb[i].double(), axb[i], t / cnt[:, None, None])
+    return {"xa": xa, "axa": axa}
+
+
+def _bracket(grid, x, periodic):
+    n = grid.numel()
+    j = torch.searchsorted(grid.double(), x)
+    j1 = j.clamp(1, n - 1)
+    lo, hi = grid[j1 - 1], grid[j1]
+    d = (hi - lo).double()
+    w = (d - x + lo.double()) / d
+    i0, i1 = j1 - 1, j1
+    first, last = j == 0, j == n
+    i0, i1, w = (torch.where(first, 0, i0), torch.where(first, 0, i1), torch.where(first, 0.0, w))
+    if not periodic:
+        return (torch.where(last, n - 1, i0), torch.where(last, n - 1, i1),
+                torch.where(last, 1.0, w))
+    gw = grid[0] + 360.0
+    d = (gw - grid[n - 1]).double()
+    ww = (d - x + grid[n - 1].double()) / d
+    wrap = last & (x <= gw.double())
+    i0 = torch.where(last, torch.where(wrap, n - 1, 0), i0)
+    i1 = torch.where(last, 0, i1)
+    return i0, i1, torch.where(last, torch.where(wrap, ww, 0.0), w)
+
+
+def _exact_obsop(case, seed):
+    d = _obsop_inputs(case, seed)
+    vc = _vcoord(case)
+    nz, k, nlat = case["nz"], case["k"], case["nlat"]
+    start, _ = _layout(nz)
+    nrec, onz, onv = case["nrec"], case["onz"], case["onv"]
+    yb = torch.empty(nrec, onz, onv, k, dtype=F64, device=DEV)
+    dep = torch.empty(nrec, onz, onv, dtype=F64, device=DEV)
+    c1, c2 = vc["c1"], vc.get("c2")
+    for r0 in range(0, nrec, 8192):
+        s = slice(r0, min(nrec, r0 + 8192))
+        a0, a1, t1 = _bracket(d["grid_lat"], d["lat"][s], False)
+        b0, b1, t2 = _bracket(d["grid_lon"], d["lon"][s], True)
+        t1, t2 = t1[:, None], t2[:, None]
+
+        def horiz(row):
+            def at(a, b):
+                col = (a + nlat * b)[:, None].expand(-1, k)
+                e = torch.arange(k, device=DEV)[None, :]
+                return d["xb"][col, row, e] + d["axb"][col, row]
+            r1 = at(a0, b0) * t1 + at(a1, b0) * (1 - t1)
+            r2 = at(a0, b1) * t1 + at(a1, b1) * (1 - t1)
+            return r1 * t2 + r2 * (1 - t2)
+
+        ps = horiz(torch.zeros(t1.shape[0], k, dtype=torch.int64, device=DEV))
+        if vc["type"] == 0:
+            half = c1 * (ps[..., None] - PTOP) + PTOP
+        else:
+            half = c1 * (vc["p0"] - PTOP) + c2 * (ps[..., None] - PTOP) + PTOP
+        full = 0.5 * (half[..., :-1] + half[..., 1:])
+        for lev in range(onz):
+            po = d["ph"][s, lev][:, None].expand(-1, k)
+            pos = (full < po[..., None]).sum(-1)
+            up, dn = (pos - 1).clamp(0, nz - 1), pos.clamp(0, nz - 1)
+            lu = torch.log(full.gather(-1, up[..., None])[..., 0])
+            ll = torch.log(full.gather(-1, dn[..., None])[..., 0])
+            same = up == dn
+            t3 = torch.where(same, 0.0, (ll - torch.log(po)) / torch.where(same, 1.0, ll - lu))
+            for v in range(onv):
+                vs = start[d["vid"][v]]
+                h = horiz(vs + up) * t3 + horiz(vs + dn) * (1 - t3)
+                mean = h.mean(1)
+                yb[s, lev, v] = h - mean[:, None]
+                dep[s, lev, v] = d["yo"][s, lev, v] - mean
+    ns = nrec * onz * onv
+    return {"lat": d["lat"].repeat_interleave(onz * onv), "lon": d["lon"].repeat_interleave(onz * onv),
+            "yb": yb.view(ns, k), "dep": dep.view(ns)}
+
+
+def _exact_cycle(case, seed):
+    atm, atm_a, xa, axa = _cycle_inputs(case, seed)
+    nz, k, nlat, nlon = case["nz"], case["k"], case["nlat"], case["nlon"]
+    n = 1 + 3 * nz
+    xb = torch.cat([t.permute(2, 1, 0, 3) for t in atm], 2).contiguous()
+    axb = torch.cat([t.permute(2, 1, 0) for t in atm_a], 2).contiguous()
+    xa, axa = xa.view(nlon, nlat, n, k), axa.view(nlon, nlat, n)
+    inside = (_grid(nlat, nlon)[0].double().abs() <= 85.0)[None, :, None]
+    full_b = xb + axb[..., None]
+    out = torch.where(inside[..., None], 0.3 * full_b + 0.7 * (xa + axa[..., None]), full_b)
+    sb = xb.square().mean(-1).sqrt()
+    sa = torch.where(inside, (out - axa[..., None]).square().mean(-1).sqrt(), sb)
+    start, lev = _layout(nz)
+    back = [out[:, :, start[v]:start[v] + lev[v]].permute(2, 1, 0, 3).contiguous()
+            for v in range(4)]
+    back_a = [axa[:, :, start[v]:start[v] + lev[v]].permute(2, 1, 0).contiguous()
+              for v in range(4)]
+    return {"xb": xb, "axb": axb, "xa_out": out, "spread_b": sb.view(-1, n),
+            "spread_a": sa.view(-1, n), "atm": back, "atm_a": back_a}
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "sweep":
+        return _exact_sweep(case, seed)
+    if kind == "obsop":
+        return _exact_obsop(case, seed)
+    if kind == "cycle":
+        return _exact_cycle(case, seed)
+    if kind == "dev":
+        nb, y, ri, dep, rl = _dev_inputs(case, seed)
+    else:
+        nb, y, ri, dep, rl = _core_inputs(case, seed)
+        if case["r4"]:
+            y, dep, rl = y.astype(np.float32), dep.astype(np.float32), rl.astype(np.float32)
+        if kind == "core":
+            nb = np.array([case["p"]])
+        nb, y, ri, dep, rl = (torch.from_numpy(t).to(DEV) for t in (nb, y, ri, dep, rl))
+    ok = torch.arange(case["p"], device=DEV)[None, :] < nb[:, None]
+    r = torch.where(ok, ri.double() * rl.double(), 0.0)
+    trans, wbar = _analysis(y.double(), r, dep.double(), 1.05)
+    if kind == "dev":
+        trans = trans.transpose(1, 2).contiguous()
+    if kind == "core":
+        trans, wbar = trans[0], wbar[0]
+    return {"trans": trans, "wbar": wbar}
