@@ -30,12 +30,6 @@ static int set_err(int code, const char *fmt, ...)
 
 const char *dida_letkf_last_error(void) { return g_err; }
 
-/* The error message of an entry point implemented in a HIP source. */
-int dk_set_error(int code, const char *msg)
-{
-    return set_err(code, "%s", msg);
-}
-
 #define HIP_TRY(expr)                                                                    \
     do {                                                                                 \
         int e_ = (int)(expr);                                                            \
@@ -1651,11 +1645,7 @@ int dida_letkf_post(int32_t k, int32_t nrow, int32_t nlat, int32_t nlon, const f
 }
 
 /* ------------------------------------------------------------------------ */
-/* Dense batched core on device pointers. */
-static _Thread_local int64_t *tl_off = NULL;
-static _Thread_local int32_t tl_off_n = 0;
-static _Thread_local int32_t tl_off_stride = 0;
-
+/* Dense batched core on device pointers: no allocation, no copy. */
 int dida_letkf_core_batch_dev(int32_t batch, int32_t max_obs, int32_t nanals,
                               const int32_t *nobsl, const double *hxens, const float *rdiaginv,
                               const double *dep, const double *rloc, double *trans,
@@ -1671,29 +1661,11 @@ int dida_letkf_core_batch_dev(int32_t batch, int32_t max_obs, int32_t nanals,
     if (!nobsl || !trans || (max_obs > 0 && (!hxens || !rdiaginv || !dep || !rloc)))
         return set_err(DIDA_ERR_ARG, "null argument");
     hipStream_t s = (hipStream_t)stream;
-    /* per-analysis offsets a * max_obs, kept per thread */
-    if (tl_off_n < batch || tl_off_stride != max_obs) {
-        if (tl_off) (void)hipFree(tl_off);
-        tl_off = NULL;
-        tl_off_n = 0;
-        int64_t *h = (int64_t *)malloc((size_t)batch * sizeof(int64_t));
-        if (!h) return set_err(DIDA_ERR_NOMEM, "host offsets");
-        for (int32_t i = 0; i < batch; ++i) h[i] = (int64_t)i * max_obs;
-        if (hipMalloc((void **)&tl_off, (size_t)batch * sizeof(int64_t)) != hipSuccess) {
-            free(h);
-            return set_err(DIDA_ERR_NOMEM, "offsets");
-        }
-        int e = (int)hipMemcpy(tl_off, h, (size_t)batch * sizeof(int64_t), hipMemcpyHostToDevice);
-        free(h);
-        if (e) return set_err(DIDA_ERR_HIP, "offset copy: %s", hipGetErrorString((hipError_t)e));
-        tl_off_n = batch;
-        tl_off_stride = max_obs;
-    }
     dk_core_args ca;
     memset(&ca, 0, sizeof ca);
     ca.k = nanals;
     ca.nanal = batch;
-    ca.offset = tl_off;
+    ca.offset = NULL; /* analysis a at a * max_obs */
     ca.nobsl = nobsl;
     ca.capacity = (int64_t)batch * max_obs;
     ca.max_p = max_obs;
@@ -1711,6 +1683,23 @@ int dida_letkf_core_batch_dev(int32_t batch, int32_t max_obs, int32_t nanals,
     ca.info = info;
     HIP_TRY(dk_letkf_core_f64(&ca, s));
     return DIDA_OK;
+}
+
+/* As dida_letkf_core_batch_dev, with the batch size its callers were promised
+ * to be refused above. */
+#define DIDA_NOALLOC_MAX_BATCH (1 << 20)
+int dida_letkf_core_batch_dev_noalloc(int32_t batch, int32_t max_obs, int32_t nanals,
+                                      const int32_t *nobsl, const double *hxens,
+                                      const float *rdiaginv, const double *dep,
+                                      const double *rloc, double *trans, double *overline_w,
+                                      double inflation_factor, int32_t gram, int32_t *info,
+                                      void *stream)
+{
+    if (batch > DIDA_NOALLOC_MAX_BATCH)
+        return set_err(DIDA_ERR_ARG, "core_batch_dev_noalloc: batch above 1048576 analyses; "
+                       "split the batch or call dida_letkf_core_batch_dev");
+    return dida_letkf_core_batch_dev(batch, max_obs, nanals, nobsl, hxens, rdiaginv, dep, rloc,
+                                     trans, overline_w, inflation_factor, gram, info, stream);
 }
 
 /* Host-pointer batch: stages through device buffers kept per thread. */

@@ -133,7 +133,7 @@ typedef struct dk_core_args {
     const int32_t *list;    /* analysis ids (NULL: aid0 + block index) */
     int32_t aid0;           /* first analysis id; trans/wbar hold id - aid0 */
     int32_t gram;           /* DK_GRAM_*: FP64 (every kernel); half-precision ones (chained) */
-    const int64_t *offset;  /* obs offset of each analysis */
+    const int64_t *offset;  /* obs offset of each analysis (NULL: id * max_p) */
     const int32_t *nobsl;   /* obs count of each analysis */
     int64_t capacity;       /* entries readable at idx/rloc; an analysis whose
                                range does not fit is treated as having no obs */
@@ -160,11 +160,12 @@ typedef struct dk_core_args {
     const double *ymax;     /* FP16X3 (chained): max_e |yb| sqrt(R^-1) per obs index */
 } dk_core_args;
 
+/* k <= 64 (dense obs only): dk_letkf_core_iter; 64 < k <= 128: a workgroup per
+ * analysis. */
 int dk_letkf_core_f64(const dk_core_args *a, void *stream);
-
-/* Sets the thread's last error message (dida_letkf_last_error) and returns
- * code; for entry points implemented in HIP sources. */
-int dk_set_error(int code, const char *msg);
+/* Dense obs blocks (idx NULL), k <= 64: one wavefront per analysis by
+ * dk_letkf_iter. */
+int dk_letkf_core_iter(const dk_core_args *a, void *stream);
 
 /* Chained analyses (64 < k <= 128): chains of chain_len consecutive
  * analyses of [aid0, aid0 + nanal), drained by nblocks persistent
@@ -330,6 +331,21 @@ int dk_letkf_wave(const dk_batched_args *a, int nblocks, void *stream);
  * trans (and wbar, info when set) as dk_letkf_core_f64.  The binned Yb rows
  * are KP = 32 or 64 values apart (zero past k), as for the batched form. */
 int dk_letkf_plain_wave(const dk_core_args *a, void *stream);
+/* FP64 analyses, k <= 64, one wavefront each, W by polynomial iteration
+ * (letkf_isqrt.h).  Of a, read: k, rho, the obs arrays (idx NULL: dense blocks
+ * of max_p obs, rows of k values; otherwise binned rows of ldy = 32 or 64
+ * values, zero past k), offset (NULL: analysis id * max_p), nobsl, max_p,
+ * capacity, base, tol / max_sweeps / predict (the Jacobi of analyses above the
+ * iteration's condition limit), info, wbar_out, phase_clk; trans_out and
+ * trans_aid0, or the state and rtps, and the vertical members. */
+typedef struct dk_iter_grid {
+    int64_t aid0, nanal;     /* analyses [aid0, aid0 + nanal) (all of them with order) */
+    const int32_t *order;    /* optional: selection tiles in processing order */
+    int32_t tj, ti;          /* with order: the tiles' shape (latitudes x longitudes) */
+    int32_t gcols, pad_;     /* set by dk_letkf_iter */
+    int64_t ngroups;
+} dk_iter_grid;
+int dk_letkf_iter(const dk_batched_args *a, const dk_iter_grid *grid, void *stream);
 /* ymax[i] = max_e |yb[i k + e]| sqrt(rinv[i]); the second form reads FP32 rows. */
 int dk_obs_ymax(int32_t nobs, int32_t k, int32_t ldy, const double *yb, const float *rinv,
                 double *ymax, void *stream);

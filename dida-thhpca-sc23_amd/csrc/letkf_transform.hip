@@ -1,15 +1,16 @@
-// LETKF transform (letkf_core, letkf_core.F90:14-233), plain FP64 form.
+// LETKF transform (letkf_core, letkf_core.F90:14-233) for 64 < k <= 128 (up to
+// 64 members: letkf_iter.hip and letkf_wave.hip).
 //
 // One workgroup (4 wavefronts) per local analysis:
-//   1. Gram C = Yhat Yhat^T on FP64 MFMA (16x16x4), Yhat = Yb sqrt(R^-1 rloc),
-//      and b = Yhat (sqrt(R^-1 rloc) dep), both accumulated straight from the
-//      gathered obs columns; the four waves split the obs and reduce in LDS.
-//   2. One-sided (Hestenes) Jacobi, resident in LDS, on M = C + (k-1)/rho I
+//   1. Gram C = Yhat Yhat^T on FP64 MFMA (16x16x4) or split half-precision
+//      MFMA, Yhat = Yb sqrt(R^-1 rloc), and b = Yhat (sqrt(R^-1 rloc) dep),
+//      accumulated straight from the gathered obs columns; the four waves
+//      split the tiles.
+//   2. One-sided (Hestenes) Jacobi in registers on M = C + (k-1)/rho I
 //      (the reference shifts the eigenvalues of C by (k-1)/rho,
-//      letkf_core.F90:110-113): column pairs of a round-robin ordering are
-//      orthogonalised in parallel until a sweep makes no rotation.  M is
-//      symmetric positive definite, so the converged columns are lambda_j v_j
-//      with every lambda_j > 0 and no separate eigenvector array is needed.
+//      letkf_core.F90:110-113).  M is symmetric positive definite, so the
+//      converged columns are lambda_j v_j with every lambda_j > 0 and no
+//      separate eigenvector array is needed.
 //   3. W = V diag(sqrt((k-1)/lambda)) V^T and wbar = V diag(1/lambda) V^T b
 //      (letkf_core.F90:129-210), trans = W + wbar 1^T.
 #include "letkf_device.h"
@@ -158,107 +159,6 @@ __device__ __forceinline__ void gram_f64_tiles(const dk_core_args& a, int64_t of
     default: gram_f64_rows<KP, 3, U>(a, off, p, sm); break;
   }
   __syncthreads();
-}
-
-// Gram + b.  KP <= 64: the obs are split across the four waves (all lower
-// tiles of C fit in one wave's accumulators) and the partial sums meet in
-// LDS.  KP = 128: the 36 lower tiles are split across the waves (tile t to
-// wave t % 4), every wave reads every obs, and wave 0 also forms b.
-template <int KP>
-__device__ __forceinline__ void gram_f64_obs(const dk_core_args& a, int64_t off, int p,
-                                             CoreSmem<KP>& sm) {
-  constexpr int NT = KP / 16;
-  constexpr int NTILE = NT * (NT + 1) / 2;
-  constexpr int LDA = CoreSmem<KP>::LDA;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r16 = lane & 15, q4 = lane >> 4;
-  const int k = a.k;
-  double4_t acc[NTILE];
-#pragma unroll
-  for (int t = 0; t < NTILE; ++t) acc[t] = double4_t{0.0, 0.0, 0.0, 0.0};
-  double bacc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) bacc[t] = 0.0;
-
-  // four chunks of 4 obs per step; obs past p read entry 0 of the analysis
-  // (in bounds: p > 0 inside the loop) with weight 0, so every load is
-  // unconditional: indices first, then the obs rows and scalars
-  constexpr int U = 4;
-  for (int c0 = wave * U; c0 * 4 < p; c0 += 4 * U) {
-    int64_t gi[U];
-    bool ok[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int o = (c0 + u) * 4 + q4;
-      ok[u] = o < p;
-      const int oc = ok[u] ? o : 0;
-      gi[u] = a.idx ? (int64_t)a.idx[off + oc] : off + oc;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    double f[U][NT], ri[U], rl[U], dp[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int oc = ok[u] ? (c0 + u) * 4 + q4 : 0;
-      ri[u] = (double)a.rinv[gi[u]];
-      rl[u] = a.rloc[off + oc];
-      dp[u] = a.dep[gi[u]];
-      const double* y = a.yb + gi[u] * k;
-#pragma unroll
-      for (int T = 0; T < NT; ++T) {
-        const int row = T * 16 + r16;
-        f[u][T] = y[row < k ? row : k - 1];
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const double rr = ok[u] ? sqrt(ri[u] * rl[u]) : 0.0;
-      const double sd = rr * dp[u];
-#pragma unroll
-      for (int T = 0; T < NT; ++T) f[u][T] = (T * 16 + r16 < k) ? f[u][T] * rr : 0.0;
-#pragma unroll
-      for (int I = 0; I < NT; ++I)
-#pragma unroll
-        for (int J = 0; J <= I; ++J)
-          acc[I * (I + 1) / 2 + J] = mfma_f64_16x16x4(f[u][I], f[u][J], acc[I * (I + 1) / 2 + J]);
-#pragma unroll
-      for (int T = 0; T < NT; ++T) bacc[T] += f[u][T] * sd;
-    }
-  }
-#pragma unroll
-  for (int T = 0; T < NT; ++T) {
-    bacc[T] += shfl_xor_d(bacc[T], 16);
-    bacc[T] += shfl_xor_d(bacc[T], 32);
-  }
-  for (int w = 0; w < 4; ++w) {
-    if (wave == w) {
-#pragma unroll
-      for (int I = 0; I < NT; ++I)
-#pragma unroll
-        for (int J = 0; J <= I; ++J) {
-          const double4_t v = acc[I * (I + 1) / 2 + J];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int i = I * 16 + 4 * r + q4, j = J * 16 + r16;
-            if (w == 0) {
-              sm.A[i + j * LDA] = v[r];
-              if (I != J) sm.A[j + i * LDA] = v[r];
-            } else {
-              sm.A[i + j * LDA] += v[r];
-              if (I != J) sm.A[j + i * LDA] += v[r];
-            }
-          }
-        }
-      if (q4 == 0) {
-#pragma unroll
-        for (int T = 0; T < NT; ++T) {
-          if (w == 0) sm.b[T * 16 + r16] = bacc[T];
-          else sm.b[T * 16 + r16] += bacc[T];
-        }
-      }
-    }
-    __syncthreads();
-  }
 }
 
 // KP = 128 Gram in half precision (batched form): Yhat = Yb sqrt(R^-1 rloc)
@@ -521,8 +421,7 @@ template <int KP, int U, int GRAM>
 __device__ __forceinline__ void gram_any(const dk_core_args& a, int64_t off, int p,
                                          CoreSmem<KP>& sm) {
   if constexpr (GRAM != DK_GRAM_FP64) gram_h16_tiles<KP, GRAM>(a, off, p, sm);
-  else if constexpr (KP > 64) gram_f64_tiles<KP, U>(a, off, p, sm);
-  else gram_f64_obs<KP>(a, off, p, sm);
+  else gram_f64_tiles<KP, U>(a, off, p, sm);
 }
 
 // One analysis by the workgroup.  vprev: eigenvectors of the previous
@@ -543,7 +442,7 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
   constexpr int LDA = CoreSmem<KP>::LDA;
   const int64_t slot = (int64_t)aid - a.aid0;
   const int k = a.k;
-  const int64_t off = a.offset[aid] - a.base;
+  const int64_t off = a.offset ? a.offset[aid] - a.base : aid * (int64_t)a.max_p;
   int p = a.nobsl[aid];
   p = p < 0 ? 0 : (p > a.max_p ? a.max_p : p);
   if (off < 0 || off + p > a.capacity) p = 0;
@@ -562,7 +461,7 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
   for (int i = tid; i < k; i += kThreads) sm.A[i + i * LDA] += a0;
   __syncthreads();
   clk.mark(DK_PHASE_GRAM);
-  if constexpr (KP == 128) {
+  {
     if (vprev) {
       // warm start A = M V_prev on MFMA: wave w owns the tiles of tile
       // columns w and w + 4 (all 8 tile rows); V_prev is read coherently
@@ -597,13 +496,8 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
   clk.mark(DK_PHASE_WARM);
 
   bool conv;
-  int sweeps;
-  if constexpr (KP == 128)
-    sweeps = jacobi_regs128<LDA, kThreads>(sm.A, sm.flag, a.tol, a.max_sweeps, a.predict != 0,
-                                           &conv);
-  else
-    sweeps = jacobi_lds<KP, LDA, kThreads>(sm.A, sm.nrm, sm.flag, a.tol, a.max_sweeps,
-                                           a.predict != 0, &conv);
+  const int sweeps = jacobi_regs128<LDA, kThreads>(sm.A, sm.flag, a.tol, a.max_sweeps,
+                                                   a.predict != 0, &conv);
   clk.mark(DK_PHASE_JACOBI);
   const int m = (k + 1) & ~1;
 
@@ -792,9 +686,7 @@ extern "C" int dk_letkf_core_f64(const dk_core_args* a, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   const int k = a->k;
   if (k < 2 || k > 128 || a->gram != DK_GRAM_FP64) return (int)hipErrorInvalidValue;
-  if (k <= 16) k_letkf_core_f64<16><<<a->nanal, kThreads, 0, s>>>(*a);
-  else if (k <= 32) k_letkf_core_f64<32><<<a->nanal, kThreads, 0, s>>>(*a);
-  else if (k <= 64) k_letkf_core_f64<64><<<a->nanal, kThreads, 0, s>>>(*a);
-  else k_letkf_core_f64<128><<<a->nanal, kThreads, 0, s>>>(*a);
+  if (k <= 64) return dk_letkf_core_iter(a, stream);
+  k_letkf_core_f64<128><<<a->nanal, kThreads, 0, s>>>(*a);
   return (int)hipGetLastError();
 }

@@ -193,26 +193,24 @@ void letkf_core_batch_r4_(const int32_t *batch, const int32_t *batch_large_matri
 
 /* Status-returning batched core on device pointers (same layout as
  * letkf_core_batch_), enqueued on `stream` (a hipStream_t, NULL = default).
- * info[batch] (optional) receives the Jacobi sweep count, -1 when the
- * eigensolve hit the sweep cap, or -2 when M or b was not finite (trans and
- * overline_w are then NaN). */
+ * info[batch] (optional) receives the solver's count (k <= 64: the steps of
+ * its polynomial iteration, or the Jacobi sweeps of an analysis whose
+ * condition number is above the iteration's limit; above: Jacobi sweeps), -1
+ * when the eigensolve hit the sweep cap, or -2 when M or b was not finite
+ * (trans and overline_w are then NaN). */
 int dida_letkf_core_batch_dev(int32_t batch, int32_t max_obs, int32_t nanals,
                               const int32_t *nobsl, const double *hxens, const float *rdiaginv,
                               const double *dep, const double *rloc, double *trans,
                               double *overline_w, double inflation_factor, int32_t gram,
                               int32_t *info, void *stream);
 
-/* The same batched core without any device allocation.  No counterpart in the
- * reference: for callers that cannot allocate device memory -- code recorded
- * in a HIP graph, tight serving loops, harnesses that forbid hipMalloc.  The
- * per-analysis obs offsets that dida_letkf_core_batch_dev stages in a buffer
- * it allocates live here in a fixed array of the library on each device (8
- * MiB, held until the process ends), written by a kernel on `stream`; no host
- * copy, no synchronisation.  batch is at most 1048576 (larger batches return
- * DIDA_ERR_ARG before anything runs).  Every call on a device shares that
- * device's array: calls that overlap on one device (unordered streams) race
- * on it; calls ordered on one stream do not.  Same arguments, layouts and
- * results as dida_letkf_core_batch_dev. */
+/* The same batched core, for callers that cannot allocate device memory (code
+ * recorded in a HIP graph, tight serving loops, harnesses that forbid
+ * hipMalloc).  No counterpart in the reference.  It allocates nothing, copies
+ * nothing to or from the host, does not synchronise and keeps no state, so
+ * calls on any streams are independent.  batch is at most 1048576 (larger
+ * batches return DIDA_ERR_ARG before anything runs).  Same arguments, layouts
+ * and results as dida_letkf_core_batch_dev. */
 int dida_letkf_core_batch_dev_noalloc(int32_t batch, int32_t max_obs, int32_t nanals,
                                       const int32_t *nobsl, const double *hxens,
                                       const float *rdiaginv, const double *dep,
