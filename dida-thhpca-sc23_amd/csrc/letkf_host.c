@@ -85,6 +85,19 @@ static int predict_of(const dida_letkf_params *p)
     return p->jacobi_predict != 0;
 }
 
+/* FP64 analyses of up to 64 members go by the polynomial iteration of
+ * dk_letkf_iter unless the caller set the Jacobi's own parameters (a tolerance,
+ * prediction, or fewer sweeps than the default), which only the Jacobi kernels
+ * honour.  Measured, Jacobi and iteration: plain sweep at 1 degree, k = 64,
+ * 31.5 and 15.3 ms; batched cubes (4, overlap 2) of the same, warm-started,
+ * 17.1 and 7.6 ms; batched vertical localisation, k = 32, 21.3 and 4.5 ms;
+ * plain sweep at 2.5 degrees, k = 20, 1.11 and 0.47 ms. */
+static int iter_of(const dida_letkf_params *p)
+{
+    return p->gram == DIDA_GRAM_FP64 && p->nanals <= 64 && p->jacobi_tol == 0.0 &&
+           p->jacobi_predict <= 0 && p->jacobi_max_sweeps >= 30;
+}
+
 static int check_params(const dida_letkf_params *p)
 {
     if (p->nanals < 2 || p->nanals > 128)
@@ -189,6 +202,7 @@ struct dida_letkf_ctx {
     int32_t chain_len, chains_per_lon, nchain, nblocks;
     int32_t ngroup;      /* 0: one cost-sorted queue; DK_XCD_GROUPS: stripes per XCD */
     int32_t chained;     /* batched form, k > 64: chained LDS analyses (vscr per CU) */
+    int32_t iter;        /* FP64 analyses by dk_letkf_iter (either form, no chains) */
     int32_t ncu;
     double *vscr;
     int32_t nchain_max;  /* chain arrays are sized for chains of one column */
@@ -402,6 +416,7 @@ int dida_letkf_create(dida_letkf_ctx **out, const dida_letkf_params *prm, int32_
     DMALLOC(c->u3, no * 3 * sizeof(double));
     DMALLOC(c->iperm, no * sizeof(int32_t));
     c->chained = prm->form == DIDA_FORM_BATCHED && k > 64;
+    c->iter = iter_of(prm);
     /* the one-wavefront kernels (batched form, and the plain form with k <= 64)
      * read binned Yb rows of 32 or 64 values, zero past k */
     c->ldy = k <= 64 && !c->chained ? (k <= 32 ? 32 : 64) : k;
@@ -801,45 +816,73 @@ static int cube_update(dida_letkf_ctx *c, const double *xb, const double *axb, d
     return DIDA_OK;
 }
 
-/* Batched form: chain queue by cost, then the persistent fused kernel. */
+/* The arguments that the one-wavefront kernels (dk_letkf_wave, dk_letkf_iter)
+ * share. */
+static void wave_args(const dida_letkf_ctx *c, dk_batched_args *b, const double *xb,
+                      const double *axb, double *xa, double *axa)
+{
+    memset(b, 0, sizeof *b);
+    b->k = c->prm.nanals;
+    b->nrow = c->prm.nrow;
+    b->nlat = c->nalat;
+    b->nlon = c->nalon;
+    b->trans_out = c->prm.cube_n > 1 ? c->trans_all : NULL;
+    b->gram = c->prm.gram;
+    b->predict = predict_of(&c->prm);
+    b->rtps = c->prm.rtps;
+    b->max_sweeps = c->prm.jacobi_max_sweeps;
+    b->max_p = c->prm.max_obs;
+    b->rtps_alpha = c->prm.rtps_alpha;
+    b->rho = c->prm.inflation_factor;
+    b->tol = jacobi_tol_of(&c->prm);
+    b->capacity = c->capacity;
+    b->offset = c->offset;
+    b->nobsl = c->nobsl;
+    b->idx = c->csr_idx;
+    b->rloc = c->csr_w;
+    b->yb = c->yb_b;
+    b->yb32 = c->yb32_b;
+    b->ldy = c->ldy;
+    b->rinv = c->rinv_b;
+    b->dep = c->dep_b;
+    b->ymax = c->ymax;
+    b->xb = xb;
+    b->axb = axb;
+    b->xa = xa;
+    b->axa = axa;
+    b->info = c->info;
+}
+
+/* Analyses [a0, a1) by dk_letkf_iter: a whole sweep in the order of the
+ * selection's tiles (most candidates first, so that the longest analyses do
+ * not start last), a part of one in grid order. */
+static int iter_launch(dida_letkf_ctx *c, const dk_batched_args *b, int64_t a0, int64_t a1,
+                       hipStream_t s)
+{
+    dk_iter_grid g;
+    memset(&g, 0, sizeof g);
+    g.aid0 = a0;
+    g.nanal = a1 - a0;
+    if (a0 == 0 && a1 == c->nsel) {
+        g.order = c->tile_order;
+        g.tj = 4;
+        g.ti = c->sel_tile == DK_SELECT_TILE_4X1 ? 1 : c->sel_tile == DK_SELECT_TILE_4X4 ? 4 : 2;
+    }
+    HIP_TRY(dk_letkf_iter(b, &g, s));
+    return DIDA_OK;
+}
+
+/* Batched form: chain queue by cost, then the persistent fused kernel (FP64
+ * analyses by the iteration: no chains). */
 static int sweep_batched(dida_letkf_ctx *c, const double *xb, const double *axb, double *xa,
                          double *axa, hipStream_t s)
 {
     dk_batched_args ba;
-    memset(&ba, 0, sizeof ba);
-    ba.k = c->prm.nanals;
-    ba.nrow = c->prm.nrow;
-    ba.nlat = c->nalat;
-    ba.nlon = c->nalon;
-    ba.trans_out = c->prm.cube_n > 1 ? c->trans_all : NULL;
+    wave_args(c, &ba, xb, axb, xa, axa);
     ba.nchain = c->nchain;
     ba.chains_per_lon = c->chains_per_lon;
     ba.chain_len = c->chain_len;
-    ba.gram = c->prm.gram;
     ba.warm_start = c->prm.warm_start ? 1 : 0;
-    ba.predict = predict_of(&c->prm);
-    ba.rtps = c->prm.rtps;
-    ba.max_sweeps = c->prm.jacobi_max_sweeps;
-    ba.max_p = c->prm.max_obs;
-    ba.rtps_alpha = c->prm.rtps_alpha;
-    ba.rho = c->prm.inflation_factor;
-    ba.tol = jacobi_tol_of(&c->prm);
-    ba.capacity = c->capacity;
-    ba.offset = c->offset;
-    ba.nobsl = c->nobsl;
-    ba.idx = c->csr_idx;
-    ba.rloc = c->csr_w;
-    ba.yb = c->yb_b;
-    ba.yb32 = c->yb32_b;
-    ba.ldy = c->ldy;
-    ba.rinv = c->rinv_b;
-    ba.dep = c->dep_b;
-    ba.ymax = c->ymax;
-    ba.xb = xb;
-    ba.axb = axb;
-    ba.xa = xa;
-    ba.axa = axa;
-    ba.info = c->info;
     ba.queue = c->chain_order;
     ba.queue_head = c->queue_head;
     if ((c->timing & 2) && c->phase_clk) {
@@ -887,6 +930,17 @@ static int sweep_batched(dida_letkf_ctx *c, const double *xb, const double *axb,
             ba.rloc = c->vw;
             ba.sel_key = c->vkey_out;
         }
+    }
+    if (c->iter) {
+        tmark(c, DIDA_STAGE_SELECT, s);
+        int rc = iter_launch(c, &ba, 0, c->nsel, s);
+        if (rc) return rc;
+        tmark(c, DIDA_STAGE_TRANSFORM, s);
+        if (ba.trans_out) {
+            HIP_TRY(cube_update(c, xb, axb, xa, axa, s));
+            tmark(c, DIDA_STAGE_UPDATE, s);
+        }
+        return DIDA_OK;
     }
     if (c->prm.gram == DIDA_GRAM_FP16X3)
         HIP_TRY(dk_obs_ymax32(c->last_nobs_pending, ba.k, c->ldy, c->yb32_b, c->rinv_b, c->ymax,
@@ -946,7 +1000,8 @@ static int sweep_batched(dida_letkf_ctx *c, const double *xb, const double *axb,
 static int core_launch(dida_letkf_ctx *c, dk_core_args *ca, hipStream_t s)
 {
     if (!c->chained)
-        return c->prm.nanals <= 64 ? dk_letkf_plain_wave(ca, s) : dk_letkf_core_f64(ca, s);
+        return c->iter ? dk_letkf_core_iter(ca, s)
+               : c->prm.nanals <= 64 ? dk_letkf_plain_wave(ca, s) : dk_letkf_core_f64(ca, s);
     dk_chain_args ch;
     ch.chain_len = c->chain_len;
     /* chains on multiples of chain_len from analysis 0 (a first partial one
@@ -981,6 +1036,20 @@ static int plain_transform(dida_letkf_ctx *c, int64_t a0, int64_t a1, int64_t ba
                            hipStream_t s)
 {
     const int k = c->prm.nanals;
+    if (c->iter && (c->prm.cube_n > 1 || !c->xa32)) {
+        /* transforms of the cubes, or analyses with their update fused */
+        dk_batched_args b;
+        wave_args(c, &b, xb, axb, xa, axa);
+        b.base = base;
+        int rc = iter_launch(c, &b, a0, a1, s);
+        if (rc) return rc;
+        tmark(c, DIDA_STAGE_TRANSFORM, s);
+        if (c->prm.cube_n > 1 && last) {
+            HIP_TRY(cube_update(c, xb, axb, xa, axa, s));
+            tmark(c, DIDA_STAGE_UPDATE, s);
+        }
+        return DIDA_OK;
+    }
     dk_core_args ca;
     memset(&ca, 0, sizeof ca);
     ca.k = k;

@@ -322,7 +322,7 @@ __global__ __launch_bounds__(64, iter_waves(KP)) void k_letkf_iter(dk_batched_ar
   const int nq = MODE == kModeVertical ? a.ncube : 1;
   const int S = gr.gcols * nq;
   const int64_t b = blockIdx.x;
-  const int64_t q = b / (8 * S) * 8 + b % 8;
+  const int64_t q = gr.group0 + b / (8 * S) * 8 + b % 8;
   const int s = (int)(b / 8 % S);
   if (q >= gr.ngroups) return;
   int64_t col;
@@ -367,21 +367,27 @@ extern "C" int dk_letkf_iter(const dk_batched_args* a, const dk_iter_grid* grid,
     g.ngroups = (g.nanal + 7) / 8;
   }
   const int64_t S = (int64_t)g.gcols * (a->ncube > 0 && !a->trans_out ? a->ncube : 1);
-  const int64_t nblocks = (g.ngroups + 7) / 8 * 8 * S;
-  if (nblocks > 0x7FFFFFFF / 64) return (int)hipErrorInvalidValue;
   hipStream_t s = (hipStream_t)stream;
-  if (a->k <= 16) return launch<16>(a, &g, nblocks, s);
-  if (a->k <= 32) return launch<32>(a, &g, nblocks, s);
-  if (a->k <= 48) return launch<48>(a, &g, nblocks, s);
-  return launch<64>(a, &g, nblocks, s);
+  // at most 2^25 blocks of 64 threads a launch (a grid holds 2^32 threads)
+  const int64_t span = (((int64_t)1 << 25) / (8 * S) > 0 ? ((int64_t)1 << 25) / (8 * S) : 1) * 8;
+  int e = 0;
+  for (g.group0 = 0; g.group0 < g.ngroups && !e; g.group0 += span) {
+    const int64_t n = g.ngroups - g.group0 < span ? g.ngroups - g.group0 : span;
+    const int64_t nblocks = (n + 7) / 8 * 8 * S;
+    e = a->k <= 16 ? launch<16>(a, &g, nblocks, s) : a->k <= 32 ? launch<32>(a, &g, nblocks, s)
+        : a->k <= 48 ? launch<48>(a, &g, nblocks, s) : launch<64>(a, &g, nblocks, s);
+  }
+  return e;
 }
 
 extern "C" int dk_letkf_core_iter(const dk_core_args* c, void* stream) {
   if (c->nanal <= 0) return 0;
-  if (c->idx || c->list) return (int)hipErrorInvalidValue;
+  if (c->list) return (int)hipErrorInvalidValue;
   dk_batched_args a;
   memset(&a, 0, sizeof a);
   a.k = c->k;
+  a.ldy = c->k <= 32 ? 32 : 64;
+  a.idx = c->idx;
   a.gram = c->gram;
   a.max_sweeps = c->max_sweeps;
   a.max_p = c->max_p;

@@ -163,8 +163,8 @@ typedef struct dk_core_args {
 /* k <= 64 (dense obs only): dk_letkf_core_iter; 64 < k <= 128: a workgroup per
  * analysis. */
 int dk_letkf_core_f64(const dk_core_args *a, void *stream);
-/* Dense obs blocks (idx NULL), k <= 64: one wavefront per analysis by
- * dk_letkf_iter. */
+/* k <= 64: one wavefront per analysis by dk_letkf_iter; dense obs blocks (idx
+ * NULL), or binned rows of 32 or 64 values. */
 int dk_letkf_core_iter(const dk_core_args *a, void *stream);
 
 /* Chained analyses (64 < k <= 128): chains of chain_len consecutive
@@ -343,7 +343,7 @@ typedef struct dk_iter_grid {
     const int32_t *order;    /* optional: selection tiles in processing order */
     int32_t tj, ti;          /* with order: the tiles' shape (latitudes x longitudes) */
     int32_t gcols, pad_;     /* set by dk_letkf_iter */
-    int64_t ngroups;
+    int64_t ngroups, group0;
 } dk_iter_grid;
 int dk_letkf_iter(const dk_batched_args *a, const dk_iter_grid *grid, void *stream);
 /* ymax[i] = max_e |yb[i k + e]| sqrt(rinv[i]); the second form reads FP32 rows. */

@@ -67,7 +67,11 @@ typedef struct dida_letkf_params {
     int32_t form;               /* DIDA_FORM_* */
     double rtps_alpha;
     int32_t gram;               /* DIDA_GRAM_* */
-    int32_t jacobi_max_sweeps;  /* eigensolver sweep cap */
+    int32_t jacobi_max_sweeps;  /* eigensolver sweep cap; below the default, with
+                                   jacobi_tol > 0 or with jacobi_predict 1, FP64
+                                   analyses of k <= 64 run the Jacobi eigensolver,
+                                   otherwise a polynomial iteration for M^(-1/2)
+                                   (at most 4 steps) that meets the same accuracy */
     double jacobi_tol;          /* rotate while |a_p.a_q| > tol |a_p||a_q|
                                    (0: 1e-13 with an FP64 Gram, 1e-8 otherwise) */
     double bin_deg;             /* obs bin size in degrees (0: automatic) */
@@ -137,10 +141,10 @@ typedef struct dida_letkf_stats {
     int32_t nobsl_max;
     int32_t nobsl_capped;       /* analyses truncated at MAX_OBS */
     int32_t nonconverged;       /* eigensolves that hit the sweep cap */
-    int32_t max_sweeps_used;
+    int32_t max_sweeps_used;    /* Jacobi sweeps, or steps of the polynomial iteration */
     int32_t capacity_overflow;  /* 1 if the selection lists did not fit */
     int32_t nonfinite;          /* analyses with a non-finite M or b (info -2) */
-    int64_t sweeps_sum;         /* Jacobi sweeps summed over converged analyses */
+    int64_t sweeps_sum;         /* sweeps or steps summed over converged analyses */
 } dida_letkf_stats;
 
 typedef struct dida_letkf_ctx dida_letkf_ctx;
