@@ -26,6 +26,10 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-command-line-argument"]
+# letkf_iter.hip holds whole matrices as MFMA results that the next MFMA and the
+# VALU read: results in VGPRs (the AGPR form spends its time moving them and
+# spills 150 registers at k = 64)
+FILE_FLAGS = {"letkf_iter.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 C_FLAGS = ["-std=c11", "-O2", "-fPIC", "-Wall", "-Wextra", f"-I{ROCM}/include"]
 
 LIB_HIP = ["letkf_select.hip", "letkf_transform.hip", "letkf_update.hip", "letkf_wave.hip",
@@ -51,7 +55,7 @@ def _obj(src):
 def _compile(src):
     path = os.path.join(CSRC, src)
     if src.endswith(".hip"):
-        _run([HIPCC, *HIP_FLAGS, "-c", path, "-o", _obj(src)])
+        _run([HIPCC, *HIP_FLAGS, *FILE_FLAGS.get(src, []), "-c", path, "-o", _obj(src)])
     else:
         _run(["gcc", *C_FLAGS, "-c", path, "-o", _obj(src)])
     return src

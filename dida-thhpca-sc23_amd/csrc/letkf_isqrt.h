@@ -30,11 +30,18 @@
 // with a spectrum far from graded), where the iteration takes 10 to 14
 // products of 160 MFMA (KP = 64) with no dependence between lanes at all.
 //
-// Layout: double4_t M[I][J], element r of lane (g = l / 16, c = l % 16) =
-// M(I*16 + 4r + g, J*16 + c), the result of mfma_f64_16x16x4.  Read as an
-// operand, M[K][J][r] is B(K*16 + 4r + g, J*16 + c), and, M being symmetric,
-// M[K][I][r] is A(I*16 + c, K*16 + 4r + g): a product needs no data movement.
-// All iterates are polynomials in M, so every product is symmetric.
+// Layout: the 16 x 16 tiles on and below the diagonal in registers, element r
+// of lane (g = l / 16, c = l % 16) of tile (I, J) = M(I*16 + 4r + g, J*16 + c),
+// the result of mfma_f64_16x16x4.  Read as operands, tile (K, J) gives
+// B(K*16 + 4r + g, J*16 + c) and, M being symmetric, tile (K, I) gives
+// A(I*16 + c, K*16 + 4r + g): the lane that holds a result holds the operand.
+// Where K is above, the operand is an element of the transposed tile below,
+// read from LDS: every product writes its off-diagonal tiles there too (all
+// iterates are polynomials in M, so every product is symmetric).  At KP = 64
+// that is 80 registers a matrix instead of 128: with whole matrices in
+// registers (and Z in LDS) the kernel spilled 416, each product waited on
+// reloads, and a 1 degree sweep took 15.3 ms instead of
+// 12.0.
 #pragma once
 
 #include "letkf_device.h"
@@ -136,89 +143,95 @@ __constant__ const IsqrtPlan kIsqrtPlan[kIsqrtPlans] = {
        {5, {2.4609375, -3.28125, 2.953125, -1.40625, 0.2734375}}}},
 };
 
-// The tiles above the diagonal from the ones below, through LDS (tile (I, J)
-// written as element (4r + g, c), read as (c, 4r + g)), two at a time.
+// The tiles on and below the diagonal of a symmetric matrix of NJ x NJ tiles.
 template <int NJ>
-__device__ __forceinline__ void mirror_lower(double4_t (&D)[NJ][NJ], double* ct) {
-  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  constexpr int NT = NJ * (NJ - 1) / 2;
-  constexpr int kI[6] = {1, 2, 2, 3, 3, 3}, kJ[6] = {0, 0, 1, 0, 1, 2};
-  static_assert(NT <= 6, "up to 4 x 4 tiles");
+struct Sym {
+  static constexpr int kTiles = NJ * (NJ + 1) / 2;
+  static constexpr int kOff = NJ * (NJ - 1) / 2;  // tiles below the diagonal
+  double4_t t[kTiles];
+  static __device__ constexpr int at(int I, int J) { return I * (I + 1) / 2 + J; }
+  static __device__ constexpr int off(int I, int J) { return I * (I - 1) / 2 + J; }
+  __device__ __forceinline__ void zero() {
 #pragma unroll
-  for (int t = 0; t < NT; t += 2) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-      if (t + u < NT)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          ct[u * 272 + (4 * r + g) * 17 + c] = D[kI[t + u]][kJ[t + u]][r];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-      if (t + u < NT)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          D[kJ[t + u]][kI[t + u]][r] = ct[u * 272 + c * 17 + 4 * r + g];
-    __syncthreads();  // read before the next tiles overwrite them
+    for (int i = 0; i < kTiles; ++i) t[i] = double4_t{0.0, 0.0, 0.0, 0.0};
   }
+  // f(I, J, r) for the elements held
+  template <class F>
+  __device__ __forceinline__ static void each(F f) {
+#pragma unroll
+    for (int I = 0; I < NJ; ++I)
+#pragma unroll
+      for (int J = 0; J <= I; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) f(I, J, r);
+  }
+};
+
+// Place of element (row, col) of a 16 x 16 tile in LDS: the columns of a row
+// are permuted so that both a tile's own rows (written) and its transpose
+// (read) touch every bank once.
+__device__ __forceinline__ int tile_at(int row, int col) { return row * 16 + (col ^ (row & 14)); }
+
+// The tiles below the diagonal to LDS (z: 256 doubles a tile).
+template <int NJ>
+__device__ __forceinline__ void publish(const Sym<NJ>& M, double* z) {
+  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  __syncthreads();  // what z held has been read
+#pragma unroll
+  for (int I = 1; I < NJ; ++I)
+#pragma unroll
+    for (int J = 0; J < I; ++J)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        z[Sym<NJ>::off(I, J) * 256 + tile_at(4 * r + g, c)] = M.t[Sym<NJ>::at(I, J)][r];
+  __syncthreads();
 }
 
-// D += A B for symmetric commuting A, B given by their operands a(K, I, r) and
-// b(K, J, r).  From 3 x 3 tiles on, the tiles on and below the diagonal only
-// (mirrored after), which saves more MFMA than the mirror costs; at 2 x 2 it
-// would save one tile of four.
-template <int NJ, class FA, class FB>
-__device__ __forceinline__ void sym_product(double4_t (&D)[NJ][NJ], FA a, FB b, double* ct) {
-  constexpr bool kLower = NJ >= 3;
+// Element (K*16 + 4r + g, J*16 + c) of M, its tiles below the diagonal in z.
+template <int NJ>
+__device__ __forceinline__ double elem(const Sym<NJ>& M, const double* z, int K, int J, int r) {
+  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  if (K >= J) return M.t[Sym<NJ>::at(K, J)][r];
+  return z[Sym<NJ>::off(J, K) * 256 + tile_at(c, 4 * r + g)];
+}
+
+// D += A B for symmetric commuting A (its tiles below the diagonal in za) and B
+// (b(K, J, r, o) = its elements, o an offset of 0 to add to LDS pointers).  o is
+// opaque to the compiler: it would otherwise keep the elements that one
+// product read for the next (48 of 512 registers, and spills).
+template <int NJ, class FB>
+__device__ __forceinline__ void sym_product(Sym<NJ>& D, const Sym<NJ>& A, const double* za,
+                                            FB b) {
+  int o = 0;
+  asm volatile("" : "+v"(o));
 #pragma unroll
   for (int K = 0; K < NJ; ++K)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      double av[NJ];
+      double av[NJ], bv[NJ];
 #pragma unroll
-      for (int I = 0; I < NJ; ++I) av[I] = a(K, I, r);
+      for (int I = 0; I < NJ; ++I) av[I] = elem<NJ>(A, za + o, K, I, r);
 #pragma unroll
-      for (int J = 0; J < NJ; ++J) {
-        const double bv = b(K, J, r);
+      for (int J = 0; J < NJ; ++J) bv[J] = b(K, J, r, o);
 #pragma unroll
-        for (int I = kLower ? J : 0; I < NJ; ++I) D[I][J] = mfma_f64_16x16x4(av[I], bv, D[I][J]);
-      }
-      // operands formed ahead of their MFMA would not fit the registers
-      if constexpr (NJ >= 4) __builtin_amdgcn_sched_barrier(0);
+      for (int I = 0; I < NJ; ++I)
+#pragma unroll
+        for (int J = 0; J <= I; ++J)
+          D.t[Sym<NJ>::at(I, J)] = mfma_f64_16x16x4(av[I], bv[J], D.t[Sym<NJ>::at(I, J)]);
     }
-  if constexpr (kLower) mirror_lower<NJ>(D, ct);
 }
 
+// Largest column sum of |M|, in every lane; NaN where there is one.
 template <int NJ>
-__device__ __forceinline__ void zero(double4_t (&D)[NJ][NJ]) {
-#pragma unroll
-  for (int I = 0; I < NJ; ++I)
-#pragma unroll
-    for (int J = 0; J < NJ; ++J) D[I][J] = double4_t{0.0, 0.0, 0.0, 0.0};
-}
-
-// f(I, J, r) for every element of a matrix.
-template <int NJ, class F>
-__device__ __forceinline__ void each(F f) {
-#pragma unroll
-  for (int I = 0; I < NJ; ++I)
-#pragma unroll
-    for (int J = 0; J < NJ; ++J)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) f(I, J, r);
-}
-
-// Largest column sum of |D|, in every lane; NaN where there is one.
-template <int NJ>
-__device__ __forceinline__ double norm1(const double4_t (&D)[NJ][NJ]) {
+__device__ __forceinline__ double norm1(const Sym<NJ>& M, const double* z) {
   double m = 0.0;
 #pragma unroll
   for (int J = 0; J < NJ; ++J) {
     double s = 0.0;
 #pragma unroll
-    for (int I = 0; I < NJ; ++I)
+    for (int K = 0; K < NJ; ++K)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s += fabs(D[I][J][r]);
+      for (int r = 0; r < 4; ++r) s += fabs(elem<NJ>(M, z, K, J, r));
     s += shfl_xor_d(s, 16);
     s += shfl_xor_d(s, 32);
     m = s > m || s != s ? s : m;  // (fmax would drop a NaN)
@@ -231,23 +244,22 @@ __device__ __forceinline__ double norm1(const double4_t (&D)[NJ][NJ]) {
   return m;
 }
 
-// T (in: M = C + a0 I, C positive semidefinite; out: Z) such that
-// M^(-1/2) = sqrt(*inv) Z.  z: KP x KP doubles of LDS for Z where three
-// matrices and Z do not fit the registers (KP = 64), else unused.  Returns the
-// steps taken, or 0 with T unchanged where M is not finite or its condition
-// bound is above kIsqrtMaxKappa.
-template <int KP>
-__device__ __forceinline__ int sym_isqrt(double4_t (&T)[KP / 16][KP / 16], double a0, double* inv,
-                                         double* ct, double* z) {
-  constexpr int NJ = KP / 16;
-  constexpr bool kZlds = KP >= 64;
+// T (in: M = C + a0 I, C positive semidefinite, published in z0; out: Z,
+// published in z2) such that M^(-1/2) = sqrt(*inv) Z.  z0, z1, z2: LDS for the
+// tiles below the diagonal of one matrix each.  Returns the steps taken, or 0
+// with T and z0 unchanged where M is not finite or its condition bound is
+// above kIsqrtMaxKappa.
+template <int NJ>
+__device__ __forceinline__ int sym_isqrt(Sym<NJ>& T, double a0, double* inv, double* z0,
+                                         double* z1, double* z2) {
+  typedef Sym<NJ> S;
   const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  typedef double4_t Mat[NJ][NJ];
-  auto opT = [&](int K, int I, int r) { return T[K][I][r]; };
-  Mat T2;
-  zero<NJ>(T2);
-  sym_product<NJ>(T2, opT, opT, ct);
-  const double kap = sqrt(norm1<NJ>(T2)) / a0 * (1.0 + 1e-12);
+  auto opT = [&](int K, int J, int r, int o) { return elem<NJ>(T, z0 + o, K, J, r); };
+  S T2;
+  T2.zero();
+  sym_product<NJ>(T2, T, z0, opT);
+  publish<NJ>(T2, z1);
+  const double kap = sqrt(norm1<NJ>(T2, z1)) / a0 * (1.0 + 1e-12);
   // (a0 outside this range could lose M^2 to underflow)
   if (!(kap <= kIsqrtMaxKappa && a0 > 1e-100 && a0 < 1e100)) return 0;
   int cls = 0;
@@ -257,70 +269,68 @@ __device__ __forceinline__ int sym_isqrt(double4_t (&T)[KP / 16][KP / 16], doubl
   const IsqrtPlan& plan = kIsqrtPlan[cls];
   const double sc = 1.0 / (a0 * kap);
   *inv = sc;
-  each<NJ>([&](int I, int J, int r) {
-    T[I][J][r] *= sc;
-    T2[I][J][r] *= sc * sc;
-  });
-  Mat Z;
+#pragma unroll
+  for (int i = 0; i < S::kTiles; ++i) {
+    T.t[i] *= sc;
+    T2.t[i] *= sc * sc;
+  }
+  publish<NJ>(T, z0);
+  publish<NJ>(T2, z1);
+  S Z;
   const int n = plan.nstep;
   for (int i = 0;; ++i) {
     const int nc = plan.step[i].nc;
     const double c0 = plan.step[i].c[0], c1 = plan.step[i].c[1], c2 = plan.step[i].c[2],
                  c3 = plan.step[i].c[3], c4 = plan.step[i].c[4];
-    Mat P;
-    each<NJ>([&](int I, int J, int r) {
-      P[I][J][r] = fma(c1, T[I][J][r], I == J && 4 * r + g == c ? c0 : 0.0);
+    auto diag = [&](int K, int J, int r, double v) {
+      return K == J && 4 * r + g == c ? v : 0.0;
+    };
+    S P;
+    S::each([&](int I, int J, int r) {
+      P.t[S::at(I, J)][r] = fma(c1, T.t[S::at(I, J)][r], diag(I, J, r, c0));
     });
     if (nc == 5) {
-      sym_product<NJ>(
-          P, [&](int K, int I, int r) { return T2[K][I][r]; },
-          [&](int K, int J, int r) {
-            return fma(c4, T2[K][J][r], fma(c3, T[K][J][r], K == J && 4 * r + g == c ? c2 : 0.0));
-          },
-          ct);
+      sym_product<NJ>(P, T2, z1, [&](int K, int J, int r, int o) {
+        return fma(c4, elem<NJ>(T2, z1 + o, K, J, r),
+                   fma(c3, elem<NJ>(T, z0 + o, K, J, r), diag(K, J, r, c2)));
+      });
     } else if (nc == 3) {
-      each<NJ>([&](int I, int J, int r) { P[I][J][r] = fma(c2, T2[I][J][r], P[I][J][r]); });
+#pragma unroll
+      for (int j = 0; j < S::kTiles; ++j) P.t[j] += c2 * T2.t[j];
     }
-    auto opP = [&](int K, int J, int r) { return P[K][J][r]; };
+    publish<NJ>(P, z1);
+    auto opP = [&](int K, int J, int r, int o) { return elem<NJ>(P, z1 + o, K, J, r); };
     const bool last = i + 1 == n;
     if (!last) {
-      Mat U;
-      zero<NJ>(U);
-      sym_product<NJ>(U, opT, opP, ct);
-      zero<NJ>(T);
-      sym_product<NJ>(T, opP, [&](int K, int J, int r) { return U[K][J][r]; }, ct);
+      S U;
+      U.zero();
+      sym_product<NJ>(U, T, z0, opP);
+      publish<NJ>(U, z0);
+      T.zero();
+      sym_product<NJ>(T, P, z1, [&](int K, int J, int r, int o) {
+        return elem<NJ>(U, z0 + o, K, J, r);
+      });
+      publish<NJ>(T, z0);
     }
     // Z <- Z P (Z = P after the first step)
-    auto z_at = [&](int I, int J, int r) { return ((I * NJ + J) * 4 + r) * 64 + lane; };
     if (i == 0) {
-      each<NJ>([&](int I, int J, int r) {
-        if constexpr (kZlds) z[z_at(I, J, r)] = P[I][J][r];
-        else Z[I][J][r] = P[I][J][r];
-      });
+      Z = P;
     } else {
-      Mat Y;
-      zero<NJ>(Y);
-      sym_product<NJ>(
-          Y,
-          [&](int K, int I, int r) {
-            if constexpr (kZlds) return z[z_at(K, I, r)];
-            else return Z[K][I][r];
-          },
-          opP, ct);
-      if (last) {
-        each<NJ>([&](int I, int J, int r) { T[I][J][r] = Y[I][J][r]; });
-        return n;
-      }
-      each<NJ>([&](int I, int J, int r) {
-        if constexpr (kZlds) z[z_at(I, J, r)] = Y[I][J][r];
-        else Z[I][J][r] = Y[I][J][r];
-      });
+      S Y;
+      Y.zero();
+      sym_product<NJ>(Y, Z, z2, opP);
+      Z = Y;
     }
+    publish<NJ>(Z, z2);
+    if (last) break;
     if (plan.step[i + 1].nc > 2) {
-      zero<NJ>(T2);
-      sym_product<NJ>(T2, opT, opT, ct);
+      T2.zero();
+      sym_product<NJ>(T2, T, z0, opT);
+      publish<NJ>(T2, z1);
     }
   }
+  T = Z;
+  return n;
 }
 
 }  // namespace dida

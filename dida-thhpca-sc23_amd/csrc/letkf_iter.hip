@@ -33,39 +33,40 @@ using namespace dida;
 
 namespace {
 
-// LDS of one analysis.  The obs staging (Gram) and the Jacobi's eigenvectors
-// are never live with the iteration's Z (KP = 64).
+// LDS of one analysis.  The obs staging (Gram), the tiles below the diagonal of
+// three matrices (iteration) and the Jacobi's eigenvectors are not live
+// together.
 template <int KP>
 struct ISmem {
   static constexpr int KPJ = KP <= 32 ? 32 : 64;  // the Jacobi's padded size
   static constexpr int LDV = KPJ + 1;
+  static constexpr int kZ = Sym<KP / 16>::kOff * 256;
   union {
     struct {
       double V[16 * LDV];
       int32_t ogi[2][64];
       double orr[2][64], ow[2][64];
+      double ct[272];
     };
-    double z[KP >= 64 ? KP * KP : 1];
+    double z[3][kZ > 0 ? kZ : 1];
   };
   double b[KPJ], f[KPJ], u[KPJ];
-  double ct[2 * 272];
 };
 
-// The FP64 Gram of one analysis: M[I][J] = C (all tiles, zero past k) and
-// sm.b.  DENSE: obs o of the analysis is row off + o of yb (k values), rinv and
+// The FP64 Gram of one analysis: M = C (zero past k) and sm.b.  DENSE: obs o of the analysis is row off + o of yb (k values), rinv and
 // dep; otherwise row idx[off + o] of the binned arrays (rows of ldy values,
 // zero past k).
 template <int KP, bool VERT, bool DENSE, class SM>
 __device__ __forceinline__ void gram_lower(const dk_batched_args& a, int64_t off, int p,
                                            double clnp, SM& sm,
-                                           double4_t (&M)[KP / 16][KP / 16]) {
+                                           Sym<KP / 16>& M) {
   constexpr int NJ = KP / 16;
   const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
   const int k = a.k;
   double bacc[NJ];
 #pragma unroll
   for (int I = 0; I < NJ; ++I) bacc[I] = 0.0;
-  zero<NJ>(M);
+  M.zero();
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<double*>(a.yb), (short)0, 0xFFFFFFFF, 0x00020000);
   const int row_shift = a.ldy == 64 ? 9 : 8;  // bytes of a binned row
@@ -99,9 +100,10 @@ __device__ __forceinline__ void gram_lower(const dk_batched_args& a, int64_t off
         bacc[I] = fma(raw[e][I], w, bacc[I]);
       }
 #pragma unroll
-      for (int J = 0; J < NJ; ++J)
+      for (int I = 0; I < NJ; ++I)
 #pragma unroll
-        for (int I = J; I < NJ; ++I) M[I][J] = mfma_f64_16x16x4(f[I], f[J], M[I][J]);
+        for (int J = 0; J <= I; ++J)
+          M.t[Sym<NJ>::at(I, J)] = mfma_f64_16x16x4(f[I], f[J], M.t[Sym<NJ>::at(I, J)]);
     }
   };
   if (p > 0) {
@@ -130,11 +132,10 @@ __device__ __forceinline__ void gram_lower(const dk_batched_args& a, int64_t off
       __syncthreads();
     }
   }
-  mirror_lower<NJ>(M, sm.ct);
   if constexpr (DENSE) {
     // rows past k repeat row k - 1
-    each<NJ>([&](int I, int J, int r) {
-      if (!(I * 16 + 4 * r + g < k && J * 16 + c < k)) M[I][J][r] = 0.0;
+    Sym<NJ>::each([&](int I, int J, int r) {
+      if (!(I * 16 + 4 * r + g < k && J * 16 + c < k)) M.t[Sym<NJ>::at(I, J)][r] = 0.0;
     });
   }
 #pragma unroll
@@ -150,7 +151,7 @@ __device__ __forceinline__ void gram_lower(const dk_batched_args& a, int64_t off
 
 // y(J*16 + c) = sum_i W(i, J*16 + c) x(i) in every lane group, x from LDS.
 template <int NJ>
-__device__ __forceinline__ void sym_apply(const double4_t (&W)[NJ][NJ], const double* x,
+__device__ __forceinline__ void sym_apply(const Sym<NJ>& W, const double* z, const double* x,
                                           double (&y)[NJ]) {
   const int g = (int)threadIdx.x >> 4;
 #pragma unroll
@@ -161,34 +162,35 @@ __device__ __forceinline__ void sym_apply(const double4_t (&W)[NJ][NJ], const do
     for (int r = 0; r < 4; ++r) {
       const double xv = x[I * 16 + 4 * r + g];
 #pragma unroll
-      for (int J = 0; J < NJ; ++J) y[J] = fma(W[I][J][r], xv, y[J]);
+      for (int J = 0; J < NJ; ++J) y[J] = fma(elem<NJ>(W, z, I, J, r), xv, y[J]);
     }
 #pragma unroll
   for (int J = 0; J < NJ; ++J) y[J] = sum_g(y[J]);
 }
 
-// W (all tiles) and wbar (sm.u, zero past k) of M and sm.b; info as the
-// entry points report it.
+// W (all tiles, zero past k) and wbar (sm.u, zero past k) of M and sm.b; info
+// as the entry points report it.
 template <int KP>
-__device__ __forceinline__ int solve(const dk_batched_args& a, ISmem<KP>& sm,
-                                     double4_t (&M)[KP / 16][KP / 16]) {
+__device__ __forceinline__ int solve(const dk_batched_args& a, ISmem<KP>& sm, Sym<KP / 16>& M,
+                                     double4_t (&W)[KP / 16][KP / 16]) {
   constexpr int NJ = KP / 16;
   constexpr int KPJ = ISmem<KP>::KPJ;
   constexpr int NJJ = KPJ / 16;
   const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
   const int k = a.k;
   const double km1 = (double)(k - 1);
+  publish<NJ>(M, sm.z[0]);
   double inv;
-  const int steps = sym_isqrt<KP>(M, km1 / a.rho, &inv, sm.ct, sm.z);
+  const int steps = sym_isqrt<NJ>(M, km1 / a.rho, &inv, sm.z[0], sm.z[1], sm.z[2]);
   if (steps > 0) {
     bool bad = false;
     double y[NJ];
-    sym_apply<NJ>(M, sm.b, y);
+    sym_apply<NJ>(M, sm.z[2], sm.b, y);
     if (g == 0)
 #pragma unroll
       for (int J = 0; J < NJ; ++J) sm.f[J * 16 + c] = y[J];
     __syncthreads();
-    sym_apply<NJ>(M, sm.f, y);
+    sym_apply<NJ>(M, sm.z[2], sm.f, y);
     const double ws = sqrt(km1 * inv);
 #pragma unroll
     for (int J = 0; J < NJ; ++J) {
@@ -196,9 +198,14 @@ __device__ __forceinline__ int solve(const dk_batched_args& a, ISmem<KP>& sm,
       bad |= !__builtin_isfinite(sm.b[J * 16 + c]) || !__builtin_isfinite(w);
       if (g == 0) sm.u[J * 16 + c] = J * 16 + c < k ? w : 0.0;
     }
-    each<NJ>([&](int I, int J, int r) {
-      M[I][J][r] = I * 16 + 4 * r + g < k && J * 16 + c < k ? M[I][J][r] * ws : 0.0;
-    });
+#pragma unroll
+    for (int I = 0; I < NJ; ++I)
+#pragma unroll
+      for (int J = 0; J < NJ; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          W[I][J][r] = I * 16 + 4 * r + g < k && J * 16 + c < k
+                           ? elem<NJ>(M, sm.z[2], I, J, r) * ws : 0.0;
     __syncthreads();
     return __any(bad) ? -2 : steps;
   }
@@ -209,13 +216,19 @@ __device__ __forceinline__ int solve(const dk_batched_args& a, ISmem<KP>& sm,
 #pragma unroll
     for (int I = 0; I < NJJ; ++I)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        w.X[J][I * 4 + r] = I < NJ && J < NJ ? M[I < NJ ? I : 0][J < NJ ? J : 0][r] : 0.0;
+      for (int r = 0; r < 4; ++r) {
+        if (I < NJ && J < NJ) w.X[J][I * 4 + r] = elem<NJ>(M, sm.z[0], I, J, r);
+        else w.X[J][I * 4 + r] = 0.0;
+      }
+  __syncthreads();  // z is read before the eigenvectors overwrite it
   bool conv;
   const int sweeps = w.jacobi(a.tol, a.max_sweeps, a.predict != 0, &conv);
   double4_t T[NJJ][NJJ], wb[NJJ];
   const bool bad = eig_transform<KPJ, DK_GRAM_FP64, false>(w, sm, km1, T, wb);
-  each<NJ>([&](int I, int J, int r) { M[I][J][r] = T[I][J][r]; });
+#pragma unroll
+  for (int I = 0; I < NJ; ++I)
+#pragma unroll
+    for (int J = 0; J < NJ; ++J) W[I][J] = T[I][J];
   if (c == 0)
 #pragma unroll
     for (int I = 0; I < NJJ; ++I)
@@ -242,17 +255,17 @@ __device__ __forceinline__ void iter_analysis(const dk_batched_args& a, int64_t 
   int lo = 0, hi = p;
   if (VERT && a.sel_key) vertical_range(a, off, p, clnp, lo, hi);
 
-  double4_t W[NJ][NJ];
-  gram_lower<KP, VERT, DENSE>(a, off + lo, hi - lo, clnp, sm, W);
+  Sym<NJ> M;
+  gram_lower<KP, VERT, DENSE>(a, off + lo, hi - lo, clnp, sm, M);
   const double a0 = (double)(k - 1) / a.rho;
 #pragma unroll
   for (int J = 0; J < NJ; ++J)
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      if (4 * r + g == c && J * 16 + c < k) W[J][J][r] += a0;
-  __syncthreads();
+      if (4 * r + g == c && J * 16 + c < k) M.t[Sym<NJ>::at(J, J)][r] += a0;
   clk.mark(DK_PHASE_GRAM);
-  const int info = solve<KP>(a, sm, W);
+  double4_t W[NJ][NJ];
+  const int info = solve<KP>(a, sm, M, W);
   clk.mark(DK_PHASE_JACOBI);
   const bool bad = info == -2;
   const double nan = __builtin_nan("");
@@ -270,22 +283,27 @@ __device__ __forceinline__ void iter_analysis(const dk_batched_args& a, int64_t 
     double wc[NJ];
 #pragma unroll
     for (int J = 0; J < NJ; ++J) wc[J] = sm.u[J * 16 + c];
-    each<NJ>([&](int I, int J, int r) {
-      const int e = I * 16 + 4 * r + g, i = J * 16 + c;
-      if (i < k && e < k) tr[i + (int64_t)e * k] = bad ? nan : W[I][J][r] + wc[J];
-    });
+#pragma unroll
+    for (int I = 0; I < NJ; ++I)
+#pragma unroll
+      for (int J = 0; J < NJ; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int e = I * 16 + 4 * r + g, i = J * 16 + c;
+          if (i < k && e < k) tr[i + (int64_t)e * k] = bad ? nan : W[I][J][r] + wc[J];
+        }
     clk.mark(DK_PHASE_TRANSFORM);
     return;
   } else {
     // T(i, e) = W + wbar 1^T on the first k rows and columns
-    double4_t wb[NJ];
 #pragma unroll
     for (int I = 0; I < NJ; ++I)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) wb[I][r] = sm.u[I * 16 + 4 * r + g];
-    each<NJ>([&](int I, int J, int r) {
-      W[I][J][r] = bad ? nan : W[I][J][r] + wb[I][r];
-    });
+      for (int r = 0; r < 4; ++r) {
+        const double wb = sm.u[I * 16 + 4 * r + g];
+#pragma unroll
+        for (int J = 0; J < NJ; ++J) W[I][J][r] = bad ? nan : W[I][J][r] + wb;
+      }
     clk.mark(DK_PHASE_TRANSFORM);
     const int32_t* rmap = VERT ? a.cube_rows + a.cube_row_off[cube] : nullptr;
     const int nr = VERT ? a.cube_row_off[cube + 1] - a.cube_row_off[cube] : a.nrow;
