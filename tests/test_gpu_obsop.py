@@ -75,3 +75,43 @@ def test_obs_operator_feeds_a_sweep(cuda, dl):
     assert st["status"] == 0 and st["nonconverged"] == 0 and st["nobsl_sum"] > 0, st
     assert torch.isfinite(xa).all() and torch.isfinite(axa).all()
     eng.close()
+
+
+# grids on both sides of 64 probes and of two rounds of them, members on both
+# sides of one a lane, members' surface pressures far apart (a level search
+# that spreads over several levels and is carried over the record's), records
+# whose levels come in no order, and obs on grid points and outside
+@pytest.mark.parametrize("nlat,nlon,k", [(1, 2, 2), (5, 63, 7), (64, 65, 64), (129, 3, 65),
+                                         (4097, 2, 3), (3, 4160, 128)])
+def test_obs_operator_grids_and_level_spread(cuda, dl, oracle, nlat, nlon, k):
+    torch = cuda
+    print(f"obs operator grid {nlat} x {nlon} k={k}", flush=True)
+    rng = np.random.default_rng(nlat + nlon + k)
+    nz, nrec, onz = 9, 300, 5
+    nrow = 1 + 2 * nz
+    glat = (-90.0 + (np.arange(nlat) + 0.5) * (180.0 / nlat)).astype(np.float32)
+    glon = (np.arange(nlon) * (360.0 / nlon)).astype(np.float32)
+    xb = rng.normal(size=(nlat * nlon, nrow, k))
+    xb[:, 0] = rng.uniform(-400.0, 400.0, (nlat * nlon, k))
+    xb -= xb.mean(axis=2, keepdims=True)
+    axb = rng.normal(size=(nlat * nlon, nrow))
+    axb[:, 0] = 950.0
+    lat, lon = rng.uniform(-90.0, 90.0, nrec), rng.uniform(0.0, 360.0, nrec)
+    lat[:20] = glat[rng.integers(0, nlat, 20)]
+    lon[10:30] = glon[rng.integers(0, nlon, 20)]
+    ph = rng.uniform(20.0, 1300.0, (nrec, onz))
+    ph[: nrec // 2].sort(axis=1)
+    yo = rng.normal(size=(nrec, onz, 2))
+    vc = {"type": 0, "c1": np.linspace(0.0, 1.0, nz + 1), "ptop": 10.0}
+    vs, vl, vid = [0, 1, 1 + nz], [1, nz, nz], [2, 0]
+    T = lambda x, dt=torch.float64: torch.tensor(np.ascontiguousarray(x), dtype=dt, device="cuda")
+    vcd = dict(vc, c1=T(vc["c1"]))
+    la, lo, yb, dep = dl.obs_operator(T(glat, torch.float32), T(glon, torch.float32), T(xb),
+                                      T(axb), 0, vcd, vs, vl, vid, T(lat), T(lon), T(ph), T(yo))
+    torch.cuda.synchronize()
+    ola, olo, oyb, odep = oracle.obs_operator(glat, glon, xb, axb, 0, vc, vs, vl, vid, lat, lon,
+                                              ph, yo)
+    assert np.array_equal(la.cpu().numpy(), ola) and np.array_equal(lo.cpu().numpy(), olo)
+    # the bars of the cases above
+    assert np.abs(yb.cpu().numpy() - oyb).max() <= 1e-12 * np.abs(oyb).max()
+    assert np.abs(dep.cpu().numpy() - odep).max() <= 1e-12 * max(np.abs(odep).max(), 1.0)
