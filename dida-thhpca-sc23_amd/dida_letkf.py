@@ -427,6 +427,15 @@ def letkf_core(hxens: np.ndarray, rdiaginv, dep, rloc, inflation: float, pflag: 
     return trans.reshape(k, k).T.copy(), wbar
 
 
+def _by_rows(trans, batch, k):
+    """(batch, i, j) arrays of the library's trans(i, j) at i + j k; large ones by
+    torch, which transposes on all host threads."""
+    if trans.size < 1 << 16:
+        return trans.reshape(batch, k, k).transpose(0, 2, 1).copy()
+    import torch
+    return torch.from_numpy(trans).view(batch, k, k).transpose(1, 2).contiguous().numpy()
+
+
 def letkf_core_batch(nobsl, hxens, rdiaginv, dep, rloc, inflation: float):
     """letkf_core_batch_ on host arrays: hxens (batch, max_obs, k)."""
     hx = np.ascontiguousarray(hxens, dtype=np.float64)
@@ -442,7 +451,7 @@ def letkf_core_batch(nobsl, hxens, rdiaginv, dep, rloc, inflation: float):
     lib().letkf_core_batch_(*[C.byref(v) for v in vals], nb.ctypes.data, hx.ctypes.data,
                             ri.ctypes.data, dp.ctypes.data, rl.ctypes.data, trans.ctypes.data,
                             wbar.ctypes.data, C.byref(rho), C.byref(pf))
-    return trans.reshape(batch, k, k).transpose(0, 2, 1).copy(), wbar.reshape(batch, k)
+    return _by_rows(trans, batch, k), wbar.reshape(batch, k)
 
 
 def letkf_core_r4(hxens: np.ndarray, rdiaginv, dep, rloc, inflation: float, pflag: int = 0):
@@ -479,7 +488,7 @@ def letkf_core_batch_r4(nobsl, hxens, rdiaginv, dep, rloc, inflation: float):
     lib().letkf_core_batch_r4_(*[C.byref(v) for v in vals], nb.ctypes.data, hx.ctypes.data,
                                ri.ctypes.data, dp.ctypes.data, rl.ctypes.data,
                                trans.ctypes.data, wbar.ctypes.data, C.byref(rho), C.byref(pf))
-    return trans.reshape(batch, k, k).transpose(0, 2, 1).copy(), wbar.reshape(batch, k)
+    return _by_rows(trans, batch, k), wbar.reshape(batch, k)
 
 
 def post(k, nrow, nlat, nlon, grid_lat, polar_lat, gamma1, gamma2, xb, axb, xa, axa, xa_out,
