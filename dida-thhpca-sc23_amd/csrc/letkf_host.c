@@ -1411,7 +1411,9 @@ int dida_letkf_autotune(dida_letkf_ctx *c, const dida_letkf_obs *o, const double
     /* 2. one chain length for all analyses, and the queue order */
     const int32_t chains[6] = {2, 4, 8, 16, 32, 64};
     const double bd1 = best_bd;
-    for (int ic = 0; ic < 6 && batched && !rc; ++ic)
+    const int chains_used = batched && !c->iter;
+    if (c->iter) best_cl = chains[2]; /* no chains: every length is the same */
+    for (int ic = 0; ic < 6 && chains_used && !rc; ++ic)
         for (int it = 0; it < 2 && !rc; ++it)
             if (!(bd1 == best_bd && chains[ic] == best_cl && it == best_tl && !best_bk))
                 TRY_LAYOUT(bd1, chains[ic], it, NULL);
@@ -1435,8 +1437,8 @@ int dida_letkf_autotune(dida_letkf_ctx *c, const dida_letkf_obs *o, const double
         const int32_t blens[7] = {1, 2, 4, 8, 16, 32, 64};
         const double bd2 = best_bd;
         const int32_t cl2 = best_cl;
-        if (!best_bk && !rc) TRY_LAYOUT(bd2, cl2, 0, bl);
-        for (int b = 0; b < DK_NBUCKET && !rc; ++b) {
+        if (!best_bk && chains_used && !rc) TRY_LAYOUT(bd2, cl2, 0, bl);
+        for (int b = 0; b < DK_NBUCKET && chains_used && !rc; ++b) {
             if (!bcount[b]) continue;
             const int32_t keep = bl[b];
             int32_t bestb = keep;
