@@ -21,10 +21,16 @@ struct WSmem {
   double b[KP];
   double f[KP];
   double u[KP];
-  int32_t ogi[2][64];  // staged obs blocks (two buffers): binned index,
-  double orr[2][64];   // sqrt(R^-1 rloc),
-  double ow[2][64];    // R^-1 rloc dep
-  double ct[16 * 17];  // a 16 x 16 tile being transposed (Gram, W), or wbar
+  // the obs staging (Gram) and the tile buffer (from its end on) are not live
+  // together
+  union {
+    struct {
+      int32_t ogi[2][64];  // staged obs blocks (two buffers): binned index,
+      double orr[2][64];   // sqrt(R^-1 rloc),
+      double ow[2][64];    // R^-1 rloc dep
+    };
+    double ct[16 * 17];  // a 16 x 16 tile being transposed (Gram, W), or wbar
+  };
 };
 
 __device__ __forceinline__ int rowA(int I, int r, int g) { return I * 16 + 4 * g + r; }

@@ -147,9 +147,12 @@ __device__ __forceinline__ int stripe_lo(int g, int n, int nlon) {
 }
 
 // One wavefront per SIMD: the fused analysis needs about 490 registers
-// (at 256, two waves a SIMD, it spills 300-700 of them and runs slower).
+// (at 256, two waves a SIMD, it spills 300-700 of them and runs slower).  Up to
+// 32 members two fit (204 to 238 registers, where unbounded instances took 257
+// and ran one: vertical localisation, k = 28, 14.1 -> 10.8 ms); bounded to
+// three they spill up to 70 (1 degree, k = 32, 4.57 -> 4.89 ms).
 template <int KP, int GRAM, int MODE>
-__global__ __launch_bounds__(64, 1) void k_letkf_wave(dk_batched_args a) {
+__global__ __launch_bounds__(64, KP == 32 ? 2 : 1) void k_letkf_wave(dk_batched_args a) {
   __shared__ WSmem<KP, true> sm;
   Wave<KP, GRAM> w;
   const int lane = threadIdx.x;
