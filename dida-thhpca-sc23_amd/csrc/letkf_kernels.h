@@ -212,8 +212,16 @@ typedef struct dk_update_args {
     float *xa32;
 } dk_update_args;
 
+/* How k_update_cols deals the columns with horizontal cubes: slat latitude
+ * segments of columns with the same covering cubes, each in plat pieces of up to
+ * clat columns; each longitude segment in plon pieces of up to clon. */
+typedef struct dk_update_grid {
+    int32_t slat, plat, clat, plon, clon;
+} dk_update_grid;
+
 int dk_update_f64(const dk_update_args *a, void *stream);
-/* The same update with FP64 MFMA, one wavefront per column (k <= 64). */
+/* The same update with FP64 MFMA, one wavefront per block of columns (k <= 64;
+ * horizontal cubes: the whole grid, ncol = nlat * nlon). */
 int dk_update_cols(const dk_update_args *a, void *stream);
 
 /* Centres of horizontal cubes: ca_lat[aj] = grid_lat[c(aj)], c(aj) the
