@@ -26,14 +26,15 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-command-line-argument"]
-# letkf_iter.hip holds whole matrices as MFMA results that the next MFMA and the
-# VALU read: results in VGPRs (the AGPR form spends its time moving them and
-# spills 150 registers at k = 64)
-FILE_FLAGS = {"letkf_iter.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# letkf_iter.hip and letkf_iter128.hip hold whole matrices as MFMA results that
+# the next MFMA and the VALU read: results in VGPRs (the AGPR form spends its time
+# moving them and spills 150 registers at k = 64)
+FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+              for f in ("letkf_iter.hip", "letkf_iter128.hip")}
 C_FLAGS = ["-std=c11", "-O2", "-fPIC", "-Wall", "-Wextra", f"-I{ROCM}/include"]
 
 LIB_HIP = ["letkf_select.hip", "letkf_transform.hip", "letkf_update.hip", "letkf_wave.hip",
-           "letkf_obsop.hip", "letkf_iter.hip"]
+           "letkf_obsop.hip", "letkf_iter.hip", "letkf_iter128.hip"]
 LIB_C = ["letkf_host.c"]
 SYNTH_HIP = ["synth.hip"]
 

@@ -88,17 +88,19 @@ static int predict_of(const dida_letkf_params *p)
     return p->jacobi_predict != 0;
 }
 
-/* FP64 analyses of up to 64 members go by the polynomial iteration of
- * dk_letkf_iter unless the caller set the Jacobi's own parameters (a tolerance,
- * prediction, or fewer sweeps than the default), which only the Jacobi kernels
- * honour.  Measured, Jacobi and iteration: plain sweep at 1 degree, k = 64,
+/* FP64 analyses go by the polynomial iteration of dk_letkf_iter and
+ * dk_letkf_iter128 unless the caller set the Jacobi's own parameters (a tolerance,
+ * prediction, fewer sweeps than the default, or above 64 members, in either form,
+ * the length of its warm-started chains), which only the Jacobi kernels honour.
+ * Measured, Jacobi and iteration: plain sweep at 1 degree, k = 64,
  * 31.5 and 15.3 ms; batched cubes (4, overlap 2) of the same, warm-started,
  * 17.1 and 7.6 ms; batched vertical localisation, k = 32, 21.3 and 4.5 ms;
  * plain sweep at 2.5 degrees, k = 20, 1.11 and 0.47 ms. */
 static int iter_of(const dida_letkf_params *p)
 {
-    return p->gram == DIDA_GRAM_FP64 && p->nanals <= 64 && p->jacobi_tol == 0.0 &&
-           p->jacobi_predict <= 0 && p->jacobi_max_sweeps >= 30;
+    const int chains = p->nanals > 64 && p->chain_len > 0;
+    return p->gram == DIDA_GRAM_FP64 && p->jacobi_tol == 0.0 && p->jacobi_predict <= 0 &&
+           p->jacobi_max_sweeps >= 30 && !chains;
 }
 
 static int check_params(const dida_letkf_params *p)
@@ -508,7 +510,7 @@ int dida_letkf_create(dida_letkf_ctx **out, const dida_letkf_params *prm, int32_
         }
         if (prm->vert_dist > 0.0) DMALLOC(c->obs_lnp, no * sizeof(double));
         /* chained analyses: one workgroup per CU, 128 x 128 eigenvectors each */
-        if (c->chained) DMALLOC(c->vscr, (size_t)ncu * 128 * 128 * sizeof(double));
+        if (c->chained && !c->iter) DMALLOC(c->vscr, (size_t)ncu * 128 * 128 * sizeof(double));
     }
     *out = c;
     return DIDA_OK;
@@ -1002,9 +1004,16 @@ static int sweep_batched(dida_letkf_ctx *c, const double *xb, const double *axb,
  * the batched form with k > 64, chains of warm-started analyses. */
 static int core_launch(dida_letkf_ctx *c, dk_core_args *ca, hipStream_t s)
 {
+    if (c->iter) {
+        if (c->chained && (c->timing & 2) && c->phase_clk) {
+            int e = (int)hipMemsetAsync(c->phase_clk, 0, DK_NPHASE * sizeof(unsigned long long), s);
+            if (e) return e;
+            ca->phase_clk = c->phase_clk;
+        }
+        return dk_letkf_core_iter(ca, s);
+    }
     if (!c->chained)
-        return c->iter ? dk_letkf_core_iter(ca, s)
-               : c->prm.nanals <= 64 ? dk_letkf_plain_wave(ca, s) : dk_letkf_core_f64(ca, s);
+        return c->prm.nanals <= 64 ? dk_letkf_plain_wave(ca, s) : dk_letkf_core_f64(ca, s);
     dk_chain_args ch;
     ch.chain_len = c->chain_len;
     /* chains on multiples of chain_len from analysis 0 (a first partial one
@@ -1039,7 +1048,7 @@ static int plain_transform(dida_letkf_ctx *c, int64_t a0, int64_t a1, int64_t ba
                            hipStream_t s)
 {
     const int k = c->prm.nanals;
-    if (c->iter && (c->prm.cube_n > 1 || !c->xa32)) {
+    if (c->iter && k <= 64 && (c->prm.cube_n > 1 || !c->xa32)) {
         /* transforms of the cubes, or analyses with their update fused */
         dk_batched_args b;
         wave_args(c, &b, xb, axb, xa, axa);
@@ -1755,7 +1764,7 @@ int dida_letkf_core_batch_dev(int32_t batch, int32_t max_obs, int32_t nanals,
     ca.trans = trans;
     ca.wbar = overline_w;
     ca.info = info;
-    HIP_TRY(dk_letkf_core_f64(&ca, s));
+    HIP_TRY(dk_letkf_core_iter(&ca, s));
     return DIDA_OK;
 }
 
@@ -2142,7 +2151,7 @@ static int core_batch_host(int32_t batch, int32_t max_obs, int32_t k, const int3
         ca.trans = (double *)res;
         ca.wbar = (double *)(res + (out[1].dst - out_at));
         ca.info = (int32_t *)(res + (info_at - out_at));
-        int e = rc ? 0 : dk_letkf_core_f64(&ca, NULL);
+        int e = rc ? 0 : dk_letkf_core_iter(&ca, NULL);
         if (e) rc = set_err(DIDA_ERR_HIP, "core: %s", hipGetErrorString((hipError_t)e));
     }
     if (!rc) {

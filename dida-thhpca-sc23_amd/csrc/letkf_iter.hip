@@ -401,6 +401,7 @@ extern "C" int dk_letkf_iter(const dk_batched_args* a, const dk_iter_grid* grid,
 extern "C" int dk_letkf_core_iter(const dk_core_args* c, void* stream) {
   if (c->nanal <= 0) return 0;
   if (c->list) return (int)hipErrorInvalidValue;
+  if (c->k > 64) return dk_letkf_iter128(c, stream);
   dk_batched_args a;
   memset(&a, 0, sizeof a);
   a.k = c->k;
@@ -424,6 +425,7 @@ extern "C" int dk_letkf_core_iter(const dk_core_args* c, void* stream) {
   a.trans_out = c->trans;
   a.trans_aid0 = c->aid0;
   a.wbar_out = c->wbar;
+  a.phase_clk = c->phase_clk;
   dk_iter_grid g;
   memset(&g, 0, sizeof g);
   g.aid0 = c->aid0;

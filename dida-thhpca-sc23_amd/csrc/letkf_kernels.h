@@ -158,13 +158,18 @@ typedef struct dk_core_args {
     int32_t ldy32;
     int32_t pad2_;
     const double *ymax;     /* FP16X3 (chained): max_e |yb| sqrt(R^-1) per obs index */
+    unsigned long long *phase_clk; /* optional (dk_letkf_core_iter) [DK_NPHASE] device
+                                      clock sums */
 } dk_core_args;
 
-/* k <= 64 (dense obs only): dk_letkf_core_iter; 64 < k <= 128: a workgroup per
- * analysis. */
+/* 64 < k <= 128: a workgroup per analysis, eigensolve by the register Jacobi. */
 int dk_letkf_core_f64(const dk_core_args *a, void *stream);
-/* k <= 64: one wavefront per analysis by dk_letkf_iter; dense obs blocks (idx
- * NULL), or binned rows of 32 or 64 values. */
+/* The same for the analyses that dk_letkf_iter128's kernel marked. */
+int dk_letkf_core_marked(const dk_core_args *a, void *stream);
+/* W by polynomial iteration.  k <= 64: one wavefront per analysis by
+ * dk_letkf_iter (dense obs blocks, idx NULL, or binned rows of 32 or 64 values);
+ * 64 < k <= 128: a workgroup per analysis by dk_letkf_iter128 (rows of k values). */
+int dk_letkf_iter128(const dk_core_args *a, void *stream);
 int dk_letkf_core_iter(const dk_core_args *a, void *stream);
 
 /* Chained analyses (64 < k <= 128): chains of chain_len consecutive

@@ -601,6 +601,17 @@ __global__ __launch_bounds__(kThreads) void k_letkf_core_f64(dk_core_args a) {
   analysis_f64<KP, 6, DK_GRAM_FP64>(a, aid, sm, nullptr, nullptr, nullptr);
 }
 
+// The analyses whose transform starts with the mark of k_letkf_iter128 (a few
+// ill-conditioned ones, as a rule none), a persistent grid looking through all.
+template <int KP>
+__global__ __launch_bounds__(kThreads) void k_letkf_core_marked(dk_core_args a) {
+  __shared__ CoreSmem<KP> sm;
+  const int64_t kk = (int64_t)a.k * a.k;
+  for (int o = blockIdx.x; o < a.nanal; o += gridDim.x)
+    if (__double_as_longlong(a.trans[o * kk]) == kMarkBits)
+      analysis_f64<KP, 6, DK_GRAM_FP64>(a, a.aid0 + o, sm, nullptr, nullptr, nullptr);
+}
+
 // Analyses [c0, c1) of chain q of a launch over [aid0, aid0 + nanal): chains
 // start at multiples of chain_len counted from analysis 0, so a launch that
 // starts inside a chain runs the rest of it as its first chain, and how a
@@ -685,8 +696,16 @@ extern "C" int dk_letkf_core_f64(const dk_core_args* a, void* stream) {
   if (a->nanal <= 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const int k = a->k;
-  if (k < 2 || k > 128 || a->gram != DK_GRAM_FP64) return (int)hipErrorInvalidValue;
-  if (k <= 64) return dk_letkf_core_iter(a, stream);
+  if (k <= 64 || k > 128 || a->gram != DK_GRAM_FP64) return (int)hipErrorInvalidValue;
   k_letkf_core_f64<128><<<a->nanal, kThreads, 0, s>>>(*a);
+  return (int)hipGetLastError();
+}
+
+extern "C" int dk_letkf_core_marked(const dk_core_args* a, void* stream) {
+  if (a->nanal <= 0) return 0;
+  if (a->k <= 64 || a->k > 128 || a->gram != DK_GRAM_FP64 || a->list)
+    return (int)hipErrorInvalidValue;
+  const int nb = a->nanal < 256 ? a->nanal : 256;
+  k_letkf_core_marked<128><<<nb, kThreads, 0, (hipStream_t)stream>>>(*a);
   return (int)hipGetLastError();
 }
