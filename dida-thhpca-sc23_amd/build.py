@@ -34,7 +34,8 @@ FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 C_FLAGS = ["-std=c11", "-O2", "-fPIC", "-Wall", "-Wextra", f"-I{ROCM}/include"]
 
 LIB_HIP = ["letkf_select.hip", "letkf_transform.hip", "letkf_update.hip", "letkf_wave.hip",
-           "letkf_obsop.hip", "letkf_iter.hip", "letkf_iter128.hip"]
+           "letkf_obsop.hip", "letkf_iter.hip", "letkf_iter128.hip",
+           "letkf_columns.hip"]
 LIB_C = ["letkf_host.c"]
 SYNTH_HIP = ["synth.hip"]
 

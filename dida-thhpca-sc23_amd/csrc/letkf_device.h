@@ -74,8 +74,9 @@ __device__ __forceinline__ double shfl_xor_d(double v, int mask) {
 // holds D[4*r + l/16][l%16] in element r (rows interleaved across the four
 // 16-lane groups; measured on gfx950).
 typedef double double4_t __attribute__((ext_vector_type(4)));
-// two doubles on an 8-byte boundary (one 16-byte access)
+// two doubles on an 8-byte boundary, four floats on a 4-byte one (16-byte accesses)
 typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
+typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ double4_t mfma_f64_16x16x4(double a, double b, double4_t c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);

@@ -816,7 +816,7 @@ static int cube_update(dida_letkf_ctx *c, const double *xb, const double *axb, d
     ua.nalon = c->nalon;
     ua.xb32 = c->xb32;
     ua.xa32 = c->xa32;
-    if (ua.k <= 64 && !ua.xa32) HIP_TRY(dk_update_cols(&ua, s));
+    if (ua.k > 64 || !ua.xa32) HIP_TRY(dk_update_cols(&ua, s));
     else HIP_TRY(dk_update_f64(&ua, s));
     return DIDA_OK;
 }
@@ -1131,7 +1131,7 @@ static int plain_transform(dida_letkf_ctx *c, int64_t a0, int64_t a1, int64_t ba
         tmark(c, DIDA_STAGE_TRANSFORM, s);
         ua.col0 = (int32_t)c0;
         ua.ncol = n;
-        if (k <= 64 && !ua.xa32) HIP_TRY(dk_update_cols(&ua, s));
+        if (k > 64 || !ua.xa32) HIP_TRY(dk_update_cols(&ua, s));
         else HIP_TRY(dk_update_f64(&ua, s));
         tmark(c, DIDA_STAGE_UPDATE, s);
     }

@@ -211,13 +211,14 @@ typedef struct dk_update_args {
      * aj + nalat ai over cube starts aj * step (latitude), ai * step
      * (longitude), each cube cube_n columns wide (clipped at the last) */
     int32_t nlat, nlon, cube_n, step, nalat, nalon;
-    /* FP32 perturbations (dk_update_f64 only): when xa32 is set, Xb' is read
+    /* FP32 perturbations (dk_update_f64, and dk_update_cols above 64 members):
+     * when xa32 is set, Xb' is read
      * from xb32 and Xa' written to xa32 instead of xb / xa */
     const float *xb32;
     float *xa32;
 } dk_update_args;
 
-/* How k_update_cols deals the columns with horizontal cubes: slat latitude
+/* How dk_update_cols deals the columns with horizontal cubes: slat latitude
  * segments of columns with the same covering cubes, each in plat pieces of up to
  * clat columns; each longitude segment in plon pieces of up to clon. */
 typedef struct dk_update_grid {
@@ -225,8 +226,9 @@ typedef struct dk_update_grid {
 } dk_update_grid;
 
 int dk_update_f64(const dk_update_args *a, void *stream);
-/* The same update with FP64 MFMA, one wavefront per block of columns (k <= 64;
- * horizontal cubes: the whole grid, ncol = nlat * nlon). */
+/* The same update with FP64 MFMA, one wavefront (k <= 64, FP64 state) or
+ * workgroup (64 < k <= 128) per block of columns; horizontal cubes: the whole
+ * grid, ncol = nlat * nlon. */
 int dk_update_cols(const dk_update_args *a, void *stream);
 
 /* Centres of horizontal cubes: ca_lat[aj] = grid_lat[c(aj)], c(aj) the

@@ -240,194 +240,6 @@ __global__ void k_chain_keys(dk_batched_args a, uint32_t* key, int32_t* id) {
   id[c] = c;
 }
 
-// Update of columns from stored transforms: a column's own (trans + (col - col0)
-// k^2) or, with horizontal cubes, the mean of the covering cubes' transforms
-// (summed in the reference's cube order: longitude starts outer, latitude
-// inner; averaging transforms equals averaging the cubes' re-centred analyses,
-// which are linear in trans).
-//
-// Bound by HBM (Xb' in, Xa' out); the transforms come from L2 and stay in
-// registers.  Columns between two consecutive starts or ends of cubes share
-// their covering cubes, so a wavefront takes a block of them (up to clat x clon
-// of one latitude and one longitude segment): the mean is formed once a block
-// instead of once a column, and the rows of neighbouring latitudes are
-// contiguous, one list of tiles of 16 rows.  Members go to the MFMA steps in
-// the order i = 16 I + 4g + r, e = 16 E + 4g + r, so that a lane's four values
-// of a tile are adjacent in trans, Xb' and Xa' (16-byte accesses).  Measured at 1
-// degree, k = 64, cubes of 4 with overlap 2: 3.27 ms with a column a wavefront
-// and 8-byte accesses, 1.57 ms (4.1 TB/s) so; bounded to 256 registers, two
-// wavefronts a SIMD, it spills 55 and takes 1.8 ms.
-struct ColSeg {
-  int start, len, a0, a1;  // columns [start, start + len), cubes a0 .. a1
-};
-// Segment q of an axis of n columns, cubes of cn columns every st.
-__device__ __forceinline__ ColSeg col_segment(int q, int n, int cn, int st, int na) {
-  const int r = cn % st;
-  const int m = r ? q >> 1 : q;
-  ColSeg s;
-  s.start = m * st + (r && (q & 1) ? r : 0);
-  s.len = min(r ? (q & 1 ? st - r : r) : st, n - s.start);
-  s.a0 = s.start - cn + 1 > 0 ? (s.start - cn + st) / st : 0;
-  s.a1 = min(s.start / st, na - 1);
-  return s;
-}
-
-template <int KP>
-__global__ __launch_bounds__(64, KP <= 32 ? 4 : KP == 48 ? 2 : 1) void k_update_cols(dk_update_args u,
-                                                                      dk_update_grid gr) {
-  constexpr int NJ = KP / 16;
-  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  const int k = u.k;
-  // four consecutive values from p on; LAST (the tile that k ends in): those
-  // from n on zero
-  auto load4 = [](auto last, const double* p, int n) {
-    double4_t v;
-    if (!last.value || n >= 4) {
-      const d2u_t a = *reinterpret_cast<const d2u_t*>(p);
-      const d2u_t b = *reinterpret_cast<const d2u_t*>(p + 2);
-      v = double4_t{a[0], a[1], b[0], b[1]};
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = r < n ? p[r] : 0.0;
-    }
-    return v;
-  };
-  const int em = 4 * (c & 3) + (c >> 2);  // the member of a tile that lane c feeds
-  const int i_last = (NJ - 1) * 16 + 4 * g;  // the lane's first member in the last tile
-  const double4_t zero = double4_t{0.0, 0.0, 0.0, 0.0};
-  double4_t T[NJ][NJ];
-#pragma unroll
-  for (int I = 0; I < NJ; ++I)
-#pragma unroll
-    for (int E = 0; E < NJ; ++E) T[I][E] = zero;
-  auto add_trans = [&](const double* tr) {
-#pragma unroll
-    for (int E = 0; E < NJ; ++E) {
-      const int e = E * 16 + em;
-      const bool in = E < NJ - 1 || e < k;
-      const double* col = tr + (int64_t)(in ? e : 0) * k;
-#pragma unroll
-      for (int I = 0; I < NJ - 1; ++I) {
-        const double4_t v = load4(std::false_type(), col + I * 16 + 4 * g, 4);
-        T[I][E] += in ? v : zero;
-      }
-      const double4_t v = load4(std::true_type(), col + i_last, k - i_last);
-      T[NJ - 1][E] += in ? v : zero;
-    }
-  };
-  int ilat = 0, nlat = 1, ilon = 0, nlon = 1;  // the block's columns
-  if (u.cube_n > 1) {
-    int b = blockIdx.x;
-    const int pa = b % gr.plat;
-    b /= gr.plat;
-    const ColSeg sa = col_segment(b % gr.slat, u.nlat, u.cube_n, u.step, u.nalat);
-    b /= gr.slat;
-    const int po = b % gr.plon;
-    const ColSeg so = col_segment(b / gr.plon, u.nlon, u.cube_n, u.step, u.nalon);
-    ilat = sa.start + pa * gr.clat;
-    nlat = min(gr.clat, sa.start + sa.len - ilat);
-    ilon = so.start + po * gr.clon;
-    nlon = min(gr.clon, so.start + so.len - ilon);
-    if (nlat <= 0 || nlon <= 0) return;
-    for (int ai = so.a0; ai <= so.a1; ++ai)
-      for (int aj = sa.a0; aj <= sa.a1; ++aj)
-        add_trans(u.trans + ((int64_t)aj + (int64_t)u.nalat * ai) * k * k);
-    const double cnt = (double)((sa.a1 - sa.a0 + 1) * (so.a1 - so.a0 + 1));
-#pragma unroll
-    for (int I = 0; I < NJ; ++I)
-#pragma unroll
-      for (int E = 0; E < NJ; ++E)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) T[I][E][r] /= cnt;
-  } else {
-    add_trans(u.trans + (int64_t)blockIdx.x * k * k);
-  }
-  const int nr = nlat * u.nrow;
-  for (int x = 0; x < nlon; ++x) {
-    const int64_t col = u.cube_n > 1 ? (int64_t)ilat + (int64_t)u.nlat * (ilon + x)
-                                     : (int64_t)u.col0 + blockIdx.x;
-    const double* xb = u.xb + col * u.nrow * k;
-    const double* axb = u.axb + col * u.nrow;
-    double* xa = u.xa + col * u.nrow * k;
-    double* axa = u.axa + col * u.nrow;
-    // Xb' and xbar of rows R0 + c, the next tile's in flight while one computes
-    auto load_rows = [&](int R0, double4_t (&v)[NJ], double& xbar) {
-      const int row = R0 + c < nr ? R0 + c : nr - 1;
-      xbar = axb[row];
-#pragma unroll
-      for (int I = 0; I < NJ - 1; ++I)
-        v[I] = load4(std::false_type(), xb + (int64_t)row * k + I * 16 + 4 * g, 4);
-      v[NJ - 1] = load4(std::true_type(), xb + (int64_t)row * k + i_last, k - i_last);
-    };
-    double4_t xl[NJ];
-    double xbar;
-    load_rows(0, xl, xbar);
-    for (int R0 = 0; R0 < nr; R0 += 16) {
-      const int row = R0 + c;
-      const bool rok = row < nr;
-      double4_t xn[NJ], D[NJ];
-      double xbarn;
-      load_rows(R0 + 16, xn, xbarn);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int E = 0; E < NJ; ++E) D[E] = zero;
-      double ssb = 0.0;
-#pragma unroll
-      for (int I = 0; I < NJ; ++I)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const double xv = xl[I][r];
-          if (u.rtps) ssb = fma(xv, xv, ssb);
-#pragma unroll
-          for (int E = 0; E < NJ; ++E) D[E] = mfma_f64_16x16x4(T[I][E][r], xv, D[E]);
-        }
-      // D[E][r]: member 16 E + 4g + r of the lane's row without xbar (members
-      // past k are zero, as their trans columns), so that the mean of the
-      // deviations does not carry xbar's rounding
-      double4_t s4 = D[0];
-#pragma unroll
-      for (int E = 1; E < NJ; ++E) s4 += D[E];
-      const double mean = sum_g((s4[0] + s4[1]) + (s4[2] + s4[3])) / (double)k;
-#pragma unroll
-      for (int E = 0; E < NJ; ++E) D[E] -= mean;
-      double fac = 1.0;
-      if (u.rtps) {
-        double4_t q4 = zero;
-#pragma unroll
-        for (int E = 0; E < NJ - 1; ++E) q4 += D[E] * D[E];
-        double ssa = (q4[0] + q4[1]) + (q4[2] + q4[3]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          ssa += i_last + r < k ? D[NJ - 1][r] * D[NJ - 1][r] : 0.0;
-        ssb = sum_g(ssb);
-        ssa = sum_g(ssa);
-        if (ssa > 0.0) fac = u.rtps_alpha * sqrt(ssb) / sqrt(ssa) + 1.0 - u.rtps_alpha;
-#pragma unroll
-        for (int E = 0; E < NJ; ++E) D[E] *= fac;
-      }
-      if (rok) {
-        double* q = xa + (int64_t)row * k;
-#pragma unroll
-        for (int E = 0; E < NJ; ++E) {
-          const int e = E * 16 + 4 * g;
-          if (E < NJ - 1 || e + 4 <= k) {
-            *reinterpret_cast<d2u_t*>(q + e) = d2u_t{D[E][0], D[E][1]};
-            *reinterpret_cast<d2u_t*>(q + e + 2) = d2u_t{D[E][2], D[E][3]};
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (e + r < k) q[e + r] = D[E][r];
-          }
-        }
-        if (g == 0) axa[row] = xbar + mean;
-      }
-#pragma unroll
-      for (int I = 0; I < NJ; ++I) xl[I] = xn[I];
-      xbar = xbarn;
-    }
-  }
-}
-
 __device__ __forceinline__ int bucket_of(int p, const dk_chain_build_args& a) {
   int b = 0;
   while (b + 1 < a.nbucket && p >= a.lo[b + 1]) ++b;
@@ -606,40 +418,6 @@ extern "C" int dk_letkf_plain_wave(const dk_core_args* c, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   if (c->k <= 32) k_letkf_plain<32><<<c->nanal, 64, 0, s>>>(a, c->aid0);
   else k_letkf_plain<64><<<c->nanal, 64, 0, s>>>(a, c->aid0);
-  return (int)hipGetLastError();
-}
-
-extern "C" int dk_update_cols(const dk_update_args* u, void* stream) {
-  if (u->ncol <= 0) return 0;
-  if (u->k < 2 || u->k > 64) return (int)hipErrorInvalidValue;
-  hipStream_t s = (hipStream_t)stream;
-  dk_update_grid gr;
-  memset(&gr, 0, sizeof gr);
-  int64_t nb = u->ncol;
-  if (u->cube_n > 1) {
-    // segments of each axis, and the largest blocks of columns that still leave
-    // 4096 wavefronts (4 a SIMD): rows of a column are a chain of tiles, so a
-    // small grid is better split than shared
-    const int st = u->step, per = u->cube_n % st ? 2 : 1;
-    gr.slat = (u->nlat + st - 1) / st * per;
-    const int slon = (u->nlon + st - 1) / st * per;
-    gr.clat = gr.clon = st;
-    auto blocks = [&] {
-      gr.plat = (st + gr.clat - 1) / gr.clat;
-      gr.plon = (st + gr.clon - 1) / gr.clon;
-      return (int64_t)gr.slat * gr.plat * slon * gr.plon;
-    };
-    while (blocks() < 4096 && gr.clat * gr.clon > 1) {
-      if (gr.clon >= gr.clat) gr.clon = (gr.clon + 1) / 2;
-      else gr.clat = (gr.clat + 1) / 2;
-    }
-    nb = blocks();
-  }
-  const unsigned n = (unsigned)nb;
-  if (u->k <= 16) k_update_cols<16><<<n, 64, 0, s>>>(*u, gr);
-  else if (u->k <= 32) k_update_cols<32><<<n, 64, 0, s>>>(*u, gr);
-  else if (u->k <= 48) k_update_cols<48><<<n, 64, 0, s>>>(*u, gr);
-  else k_update_cols<64><<<n, 64, 0, s>>>(*u, gr);
   return (int)hipGetLastError();
 }
 
