@@ -42,10 +42,17 @@ struct JacobiXbuf {
   int32_t id[64];
 };
 
+// v of the lane that DPP control CTRL names, for controls that give every lane a
+// valid source (quad permutations, rotations and mirrors): with bound_ctrl set
+// nothing of the old value remains, so no register is cleared before each move (a
+// seventh of the instructions of a round otherwise).
+template <int CTRL>
+__device__ __forceinline__ int dpp_u(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+}
 template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
+  const int lo = dpp_u<CTRL>(__double2loint(v)), hi = dpp_u<CTRL>(__double2hiint(v));
   return __hiloint2double(hi, lo);
 }
 // sum over the eight lanes of a group (quad_perm [1,0,3,2], [2,3,0,1], then
@@ -62,7 +69,7 @@ __device__ __forceinline__ double oct_sum(double v) {
 template <int V>
 __device__ __forceinline__ unsigned lane_xor_u(unsigned v) {
   if constexpr (V == 8) {
-    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false);
+    return (unsigned)dpp_u<0x128>((int)v);
   } else if constexpr (V == 16) {
     const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
     return (threadIdx.x & 16) ? r[0] : r[1];
