@@ -98,6 +98,9 @@ struct Jacobi128 {
     double nrm, sc, isc;
   };
   ColSt tp, bt;
+  __device__ __forceinline__ static ColSt pick(bool a, const ColSt& x, const ColSt& y) {
+    return ColSt{a ? x.nrm : y.nrm, a ? x.sc : y.sc, a ? x.isc : y.isc};
+  }
 
   template <int P, int Q>
   __device__ __forceinline__ double dot() const {
@@ -176,8 +179,8 @@ struct Jacobi128 {
     const bool second = (threadIdx.x & 4) != 0;
     const ColSt mt{dpp_d<0x141>(tp.nrm), dpp_d<0x141>(tp.sc), dpp_d<0x141>(tp.isc)};
     const ColSt mb{dpp_d<0x141>(bt.nrm), dpp_d<0x141>(bt.sc), dpp_d<0x141>(bt.isc)};
-    if (second) tp = mb;
-    else bt = mt;
+    tp = pick(second, mb, tp);
+    bt = pick(second, bt, mt);
   }
   // the pair state at a sweep's start (lanes 0-3: slots 0, 1; 4-7: 2, 3)
   __device__ __forceinline__ void state_start() {
@@ -307,25 +310,29 @@ struct Jacobi128 {
       xswap_st_lane<32>(first);
     } else {
       const int qh = sub >> 2;  // the half's pair: (0, 1) or (2, 3)
+      // (the state by value: a choice between bt and tp in memory would keep
+      // both there, two scratch loads in the chain of every round)
+      const ColSt out = pick(first, bt, tp);
       if (first) {
         put<1>(xb, gp, sub, 0);
         put<3>(xb, gp, sub, 1);
-        put_st(xb, gp, sub, qh, bt);
       } else {
         put<0>(xb, gp, sub, 0);
         put<2>(xb, gp, sub, 1);
-        put_st(xb, gp, sub, qh, tp);
       }
+      put_st(xb, gp, sub, qh, out);
       __syncthreads();
       if (first) {
         get<1>(xb, gp ^ d, sub, 0);
         get<3>(xb, gp ^ d, sub, 1);
-        get_st(xb, gp ^ d, qh, bt);
       } else {
         get<0>(xb, gp ^ d, sub, 0);
         get<2>(xb, gp ^ d, sub, 1);
-        get_st(xb, gp ^ d, qh, tp);
       }
+      ColSt in;
+      get_st(xb, gp ^ d, qh, in);
+      bt = pick(first, in, bt);
+      tp = pick(first, tp, in);
       __syncthreads();
     }
   }

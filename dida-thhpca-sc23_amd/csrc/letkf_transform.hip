@@ -36,6 +36,16 @@ struct CoreSmem {
   int flag[4];
 };
 
+// threadIdx.x, opaque: what a phase derives from it (addresses, masks) is formed in
+// that phase of each analysis.  Hoisted out of the loop over the analyses of a
+// chain it took the Jacobi's registers (its state went through scratch, two loads
+// in the dependent chain of every round).
+__device__ __forceinline__ int phase_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // KP = 128 Gram: wave W owns the lower tiles of tile rows W and NT-1-W
 // (9 tiles each, fixed at compile time); every wave reads every obs.  Obs go
 // in stages of U steps of 4 (lane group q4 takes obs 4u + q4 of a step): the
@@ -48,7 +58,7 @@ __device__ __forceinline__ void gram_f64_rows(const dk_core_args& a, int64_t off
   constexpr int IA = W, IB = NT - 1 - W;  // IA < IB
   constexpr int NF = IB + 1;              // tile rows this wave reads
   constexpr int LDA = CoreSmem<KP>::LDA;
-  const int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4;
+  const int lane = phase_tid() & 63, r16 = lane & 15, q4 = lane >> 4;
   const int k = a.k;
   double4_t accA[IA + 1], accB[IB + 1];
 #pragma unroll
@@ -196,7 +206,7 @@ __device__ __forceinline__ void gram_h16_rows(const dk_core_args& a, int64_t off
   constexpr int LDA = CoreSmem<KP>::LDA;
   static_assert(sizeof(H16Stage<KP, hvec>) <= sizeof(sm.A), "staging fits in A");
   H16Stage<KP, hvec>& st = *reinterpret_cast<H16Stage<KP, hvec>*>(sm.A);
-  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int tid = phase_tid(), lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int rq = tid & 31, og = tid >> 5;  // staging rows 4 rq.., obs octet og
   const int k = a.k;
   const bool rows_ok = 4 * rq < k;
@@ -446,8 +456,7 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
   int p = a.nobsl[aid];
   p = p < 0 ? 0 : (p > a.max_p ? a.max_p : p);
   if (off < 0 || off + p > a.capacity) p = 0;
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63, r16 = lane & 15, q4 = lane >> 4;
+  const int tid0 = threadIdx.x;
 
   // the previous analysis of a chain may still be reading A (its W tiles)
   __syncthreads();
@@ -458,7 +467,7 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
   // M = C + (k-1)/rho I on the first k diagonal entries (letkf_core.F90:110-113
   // applies the shift to the eigenvalues; M is positive definite, so every
   // converged column is a non-null lambda_j v_j)
-  for (int i = tid; i < k; i += kThreads) sm.A[i + i * LDA] += a0;
+  for (int i = tid0; i < k; i += kThreads) sm.A[i + i * LDA] += a0;
   __syncthreads();
   clk.mark(DK_PHASE_GRAM);
   {
@@ -466,6 +475,8 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
       // warm start A = M V_prev on MFMA: wave w owns the tiles of tile
       // columns w and w + 4 (all 8 tile rows); V_prev is read coherently
       // with L2 (another analysis of this workgroup wrote it)
+      const int tid = phase_tid();
+      const int wave = tid >> 6, lane = tid & 63, r16 = lane & 15, q4 = lane >> 4;
       double4_t d[NT][2];
 #pragma unroll
       for (int I = 0; I < NT; ++I) d[I][0] = d[I][1] = double4_t{0.0, 0.0, 0.0, 0.0};
@@ -500,6 +511,8 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
                                                    a.predict != 0, &conv);
   clk.mark(DK_PHASE_JACOBI);
   const int m = (k + 1) & ~1;
+  const int tid = phase_tid();
+  const int wave = tid >> 6, lane = tid & 63, r16 = lane & 15, q4 = lane >> 4;
 
   // exact column norms: alpha_j = lambda_j^2, lambda_j eigenvalues of M
   int nonfinite = 0;
