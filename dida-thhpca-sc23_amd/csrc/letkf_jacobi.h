@@ -63,16 +63,18 @@ __device__ __forceinline__ double oct_sum(double v) {
   return v + dpp_d<0x141>(v);
 }
 
-// v of lane l ^ V (V = 8: DPP row_ror:8 inside each 16-lane row; V = 16, 32:
-// v_permlane16/32_swap of v with itself, whose first result holds the value
-// of the lower row (lanes l & ~V) and the second that of the upper one)
+// v of lane l ^ V.  V = 8: DPP row_ror:8 inside each 16-lane row, one VALU
+// instruction (1 degree, k = 128: 165.7 ms a sweep, against 171.6 by ds_swizzle).
+// V = 16: ds_swizzle, one LDS instruction (172.2 by v_permlane16_swap, which takes
+// a copy, the swap and a select).  V = 32: v_permlane32_swap of v with itself,
+// whose first result holds the value of the lower lanes (l & ~V) and the second
+// that of the upper ones (169.0 by ds_bpermute).
 template <int V>
 __device__ __forceinline__ unsigned lane_xor_u(unsigned v) {
   if constexpr (V == 8) {
     return (unsigned)dpp_u<0x128>((int)v);
   } else if constexpr (V == 16) {
-    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    return (threadIdx.x & 16) ? r[0] : r[1];
+    return (unsigned)__builtin_amdgcn_ds_swizzle((int)v, 0x1F | (16 << 10));
   } else {
     static_assert(V == 32, "lane xor of 8, 16 or 32");
     const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
