@@ -82,6 +82,20 @@ __device__ __forceinline__ double4_t mfma_f64_16x16x4(double a, double b, double
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// v of the lane that DPP control CTRL names, for controls that give every lane a
+// valid source (quad permutations, rotations and mirrors): with bound_ctrl set
+// nothing of the old value remains, so no register is cleared before each move (a
+// seventh of the instructions of a round otherwise).
+template <int CTRL>
+__device__ __forceinline__ int dpp_u(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const int lo = dpp_u<CTRL>(__double2loint(v)), hi = dpp_u<CTRL>(__double2hiint(v));
+  return __hiloint2double(hi, lo);
+}
+
 // v of the lane whose byte address (4 * lane) is addr
 __device__ __forceinline__ double bperm_d(int addr, double v) {
   const int lo = __builtin_amdgcn_ds_bpermute(addr, __double2loint(v));

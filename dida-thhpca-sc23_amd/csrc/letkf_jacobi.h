@@ -42,19 +42,6 @@ struct JacobiXbuf {
   int32_t id[64];
 };
 
-// v of the lane that DPP control CTRL names, for controls that give every lane a
-// valid source (quad permutations, rotations and mirrors): with bound_ctrl set
-// nothing of the old value remains, so no register is cleared before each move (a
-// seventh of the instructions of a round otherwise).
-template <int CTRL>
-__device__ __forceinline__ int dpp_u(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-  const int lo = dpp_u<CTRL>(__double2loint(v)), hi = dpp_u<CTRL>(__double2hiint(v));
-  return __hiloint2double(hi, lo);
-}
 // sum over the eight lanes of a group (quad_perm [1,0,3,2], [2,3,0,1], then
 // row_half_mirror); every lane of the group gets the same bits
 __device__ __forceinline__ double oct_sum(double v) {

@@ -86,12 +86,12 @@ __device__ __forceinline__ void split_g(double v, double& v0, double& v1) {
   v1 = __hiloint2double(b[1], a[1]);
 }
 
-// v of lane (l ^ 1), same 16-lane row (ds_swizzle, bit mode: and 0x1f, xor 1)
-__device__ __forceinline__ double swz_xor1(double v) {
-  const int lo = __builtin_amdgcn_ds_swizzle(__double2loint(v), 0x1F | (1 << 10));
-  const int hi = __builtin_amdgcn_ds_swizzle(__double2hiint(v), 0x1F | (1 << 10));
-  return __hiloint2double(hi, lo);
-}
+// v of lane l ^ 1, by DPP quad_perm [1,0,3,2]: one VALU instruction (by ds_swizzle
+// the next round's dot products waited for the LDS: 0.5 degree, k = 64: 78.8 ms a
+// sweep, 76.3 so).  The moves by other bits stay with ds_bpermute: a DPP variant
+// of each bit (two moves for bit 4) took 79.3 ms, the branches between them
+// shuffling registers.
+__device__ __forceinline__ double row_xor1(double v) { return dpp_d<0xB1>(v); }
 // Metadata of one 64-obs block of an analysis, lane l holding obs base + l:
 // binned index, sqrt(R^-1 rloc) and R^-1 rloc dep.  Entries past p take the
 // index of obs 0 and zero weights, so every load is unconditional and in
@@ -679,9 +679,9 @@ struct Wave {
     cross(tp.isc, bt.isc);
   }
   __device__ __forceinline__ void bt_xor1() {
-    bt.nrm = swz_xor1(bt.nrm);
-    bt.sc = swz_xor1(bt.sc);
-    bt.isc = swz_xor1(bt.isc);
+    bt.nrm = row_xor1(bt.nrm);
+    bt.sc = row_xor1(bt.sc);
+    bt.isc = row_xor1(bt.isc);
   }
   __device__ __forceinline__ void bt_perm(int addr) {
     bt.nrm = bperm_d(addr, bt.nrm);
@@ -702,7 +702,7 @@ struct Wave {
   template <int J>
   __device__ __forceinline__ void x_xor1() {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) X[J][q] = swz_xor1(X[J][q]);
+    for (int q = 0; q < NQ; ++q) X[J][q] = row_xor1(X[J][q]);
   }
   template <int J>
   __device__ __forceinline__ void x_perm(int addr) {
@@ -723,10 +723,10 @@ struct Wave {
   template <int J>
   __device__ __forceinline__ void move_xor1() {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) X[J][q] = swz_xor1(X[J][q]);
-    nrm[J] = swz_xor1(nrm[J]);
-    sc[J] = swz_xor1(sc[J]);
-    isc[J] = swz_xor1(isc[J]);
+    for (int q = 0; q < NQ; ++q) X[J][q] = row_xor1(X[J][q]);
+    nrm[J] = row_xor1(nrm[J]);
+    sc[J] = row_xor1(sc[J]);
+    isc[J] = row_xor1(isc[J]);
   }
   // Column J takes the column J of the lane at byte address addr.
   template <int J>
