@@ -838,9 +838,13 @@ struct Wave {
         split_g(bt.sc, sc[2], sc[1]);
       } else {
         for (int G = KP / 2; G >= 1; G >>= 1) {
-          for (int r = 0; r < G; ++r) {
+          // (r + 1) odd: the bottom of lane l ^ 1
+          for (int r = 0; r < G; r += 2) {
             round<0, 1, 0, 1>(tol2, tolp, rotated, big);
-            if (r + 1 < G) move_perm<1>((lane ^ ((r + 1) & -(r + 1))) << 2);
+            if (G == 1) break;
+            move_xor1<1>();
+            round<0, 1, 0, 1>(tol2, tolp, rotated, big);
+            if (r + 2 < G) move_perm<1>((lane ^ ((r + 2) & -(r + 2))) << 2);
           }
           if (G > 1) {
             const int d = G >> 1;
