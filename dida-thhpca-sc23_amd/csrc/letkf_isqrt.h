@@ -14,9 +14,9 @@
 // fewest products that ends with e below 2^-56.
 //
 // kappa: the smallest eigenvalue of M = C + a0 I is at least a0 (C has no
-// negative one), the largest at most sqrt(|| M^2 ||_1), one product that the
-// first step needs anyway.  The iteration's own error grows with kappa
-// (relative error in the 2-norm against 40-digit arithmetic, 64 x 64: 7e-16 at
+// negative one), the largest at most sqrt(|| M^2 ||_1) and (trace M^4)^(1/4),
+// from one product that the first step needs anyway.  The iteration's own error
+// grows with kappa (relative error in the 2-norm against 40-digit arithmetic, 64 x 64: 7e-16 at
 // kappa 10, 3e-15 at 100, 3e-14 at 1300, 6e-14 at 3200; Jacobi with tolerance
 // 1e-13: 2e-13 throughout) and would pass the Jacobi's at some 10 000; above
 // kIsqrtMaxKappa an analysis takes the Jacobi.  T <- P (T P) has the smallest
@@ -244,6 +244,21 @@ __device__ __forceinline__ double norm1(const Sym<NJ>& M, const double* z) {
   return m;
 }
 
+// || M ||_F^2 (trace M^2) in every lane.
+template <int NJ>
+__device__ __forceinline__ double frob2(const Sym<NJ>& M) {
+  double d = 0.0, f = 0.0;
+  Sym<NJ>::each([&](int I, int J, int r) {
+    const double v = M.t[Sym<NJ>::at(I, J)][r];
+    if (I == J) d = fma(v, v, d);
+    else f = fma(v, v, f);
+  });
+  d = fma(2.0, f, d);
+#pragma unroll
+  for (int x = 1; x < 64; x <<= 1) d += shfl_xor_d(d, x);
+  return d;
+}
+
 // T (in: M = C + a0 I, C positive semidefinite, published in z0; out: Z,
 // published in z2) such that M^(-1/2) = sqrt(*inv) Z.  z0, z1, z2: LDS for the
 // tiles below the diagonal of one matrix each.  Returns the steps taken, or 0
@@ -259,7 +274,16 @@ __device__ __forceinline__ int sym_isqrt(Sym<NJ>& T, double a0, double* inv, dou
   T2.zero();
   sym_product<NJ>(T2, T, z0, opT);
   publish<NJ>(T2, z1);
-  const double kap = sqrt(norm1<NJ>(T2, z1)) / a0 * (1.0 + 1e-12);
+  double top = sqrt(norm1<NJ>(T2, z1));
+  if constexpr (NJ > 2) {
+    // the tighter bound saves up to two products (1 degree, k = 64: 11.43 -> 11.33
+    // ms a sweep); up to 32 members its reduction costs what it saves (vertical
+    // localisation, k = 32: 3.90 and 3.94 ms)
+    // (below 1e-70 the trace of M^4 could underflow)
+    const double n4 = sqrt(sqrt(frob2<NJ>(T2)));
+    top = n4 < top && a0 > 1e-70 ? n4 : top;
+  }
+  const double kap = top / a0 * (1.0 + 1e-12);
   // (a0 outside this range could lose M^2 to underflow)
   if (!(kap <= kIsqrtMaxKappa && a0 > 1e-100 && a0 < 1e100)) return 0;
   int cls = 0;

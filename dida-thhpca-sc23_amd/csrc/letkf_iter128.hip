@@ -262,7 +262,8 @@ struct Part {
     }
     const double n1 = sqrt(m);
     const double n4 = sqrt(sqrt((sm.red[0] + sm.red[1]) + (sm.red[2] + sm.red[3])));
-    return (n4 < n1 ? n4 : n1) / a0 * (1.0 + 1e-12);
+    // (below 1e-70 the trace of M^4 could underflow)
+    return (n4 < n1 && a0 > 1e-70 ? n4 : n1) / a0 * (1.0 + 1e-12);
   }
 
   // Gram and iteration: Z at sm.z[0] with M^(-1/2) = sqrt(*inv) Z, and the steps

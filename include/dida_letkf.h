@@ -68,16 +68,17 @@ typedef struct dida_letkf_params {
     double rtps_alpha;
     int32_t gram;               /* DIDA_GRAM_* */
     int32_t jacobi_max_sweeps;  /* eigensolver sweep cap; below the default, with
-                                   jacobi_tol > 0 or with jacobi_predict 1, FP64
-                                   analyses of k <= 64 run the Jacobi eigensolver,
-                                   otherwise a polynomial iteration for M^(-1/2)
-                                   (at most 4 steps) that meets the same accuracy */
+                                   jacobi_tol > 0, with jacobi_predict 1 or, above
+                                   64 members, with chain_len > 0, FP64 analyses
+                                   run the Jacobi eigensolver, otherwise a
+                                   polynomial iteration for M^(-1/2) (at most 4
+                                   steps) that meets the same accuracy */
     double jacobi_tol;          /* rotate while |a_p.a_q| > tol |a_p||a_q|
                                    (0: 1e-13 with an FP64 Gram, 1e-8 otherwise) */
     double bin_deg;             /* obs bin size in degrees (0: automatic) */
     int32_t chain_len;          /* batched form: adjacent columns per work item,
                                    each warm-starting the next one's eigensolve
-                                   (0: automatic) */
+                                   (0: automatic; see jacobi_max_sweeps) */
     int32_t warm_start;         /* batched form: 1 to warm-start along chains */
     int32_t jacobi_predict;     /* 1 ends the eigensolve after a sweep whose largest
                                    |a_p.a_q|^2 / (|a_p|^2 |a_q|^2) is <= tol (the
