@@ -92,10 +92,12 @@ static int predict_of(const dida_letkf_params *p)
  * dk_letkf_iter128 unless the caller set the Jacobi's own parameters (a tolerance,
  * prediction, fewer sweeps than the default, or above 64 members, in either form,
  * the length of its warm-started chains), which only the Jacobi kernels honour.
- * Measured, Jacobi and iteration: plain sweep at 1 degree, k = 64,
- * 31.5 and 15.3 ms; batched cubes (4, overlap 2) of the same, warm-started,
- * 17.1 and 7.6 ms; batched vertical localisation, k = 32, 21.3 and 4.5 ms;
- * plain sweep at 2.5 degrees, k = 20, 1.11 and 0.47 ms. */
+ * Measured, Jacobi and iteration: plain sweep at 1 degree, k = 64, 32.9 and 11.3
+ * ms; batched cubes (4, overlap 2) of the same 17.1 and 5.2 ms (its update 1.7 of
+ * the difference); batched vertical localisation, k = 32, 21.3 and 3.9 ms; plain
+ * sweep at 2.5 degrees, k = 20, 1.11 and 0.43 ms; batched, 80 x 160 columns, k =
+ * 82, 61.3 and 4.5 ms.  (Split half-precision Grams keep the Jacobi, whose
+ * prediction sets the last digits of their results.) */
 static int iter_of(const dida_letkf_params *p)
 {
     const int chains = p->nanals > 64 && p->chain_len > 0;

@@ -1,5 +1,7 @@
-// LETKF transform (letkf_core, letkf_core.F90:14-233) for 64 < k <= 128 (up to
-// 64 members: letkf_iter.hip and letkf_wave.hip).
+// LETKF transform (letkf_core, letkf_core.F90:14-233) for 64 < k <= 128 by the
+// register Jacobi: split half-precision Grams, callers that set the Jacobi's
+// parameters and ill-conditioned analyses (other FP64 analyses: letkf_iter128.hip;
+// up to 64 members: letkf_iter.hip and letkf_wave.hip).
 //
 // One workgroup (4 wavefronts) per local analysis:
 //   1. Gram C = Yhat Yhat^T on FP64 MFMA (16x16x4) or split half-precision
