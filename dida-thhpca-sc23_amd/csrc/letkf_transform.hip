@@ -35,6 +35,7 @@ struct CoreSmem {
   double sh[KP];
   double u[KP];
   double wb[KP];
+  double tb[4][16 * 17];  // a tile of W on its way to its transpose, per wavefront
   int flag[4];
 };
 
@@ -575,15 +576,18 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
   }
   __syncthreads();
 
-  // W = (A diag(sg)) A^T on MFMA, written with wbar as trans.  The tile of
-  // trans rows I, columns I2 is formed as W(I2 block, I block), whose result
-  // layout puts 16 consecutive rows of a trans column in 16 lanes (W is
-  // symmetric), so the stores are whole 128-byte lines.
+  // W = (A diag(sg)) A^T on MFMA, written with wbar as trans: W is symmetric, so
+  // the tiles (I, I2), I2 <= I, only.  A tile is formed as W(I2 block, I block),
+  // whose result layout puts 16 consecutive rows of a trans column in 16 lanes,
+  // and goes through LDS for its transpose, so the stores are whole 128-byte
+  // lines.  (All 64 tiles: 1 degree, k = 128, 165.5 ms a sweep, 163.3 so.)
   double* trans = a.trans + slot * k * k;
   // (columns past m are zero and sg is zero there, so the contraction runs
   // over all KP columns at compile-time trip counts, in two chains)
-  for (int t = wave; t < NT * NT; t += 4) {
-    const int I = t / NT, I2 = t % NT;
+  double* tb = sm.tb[wave];
+  for (int t = wave, I = 0; t < NT * (NT + 1) / 2; t += 4) {
+    while ((I + 1) * (I + 2) / 2 <= t) ++I;
+    const int I2 = t - I * (I + 1) / 2;
     double4_t d = double4_t{0.0, 0.0, 0.0, 0.0}, d1 = d;
 #pragma unroll
     for (int j0 = 0; j0 < KP; j0 += 8) {
@@ -594,12 +598,22 @@ __device__ bool analysis_f64(const dk_core_args& a, int aid, CoreSmem<KP>& sm,
                             sm.A[I * 16 + r16 + jb * LDA], d1);
     }
     d += d1;
-    // d[r] = W(I2*16 + 4r + q4, I*16 + r16) = W(i, i2)
+    // d[r] = W(I2*16 + 4r + q4, I*16 + r16) = W(i, i2); its transpose through LDS
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = I * 16 + r16, i2 = I2 * 16 + 4 * r + q4;
       if (i < k && i2 < k) trans[i + (int64_t)i2 * k] = bad ? nan : d[r] + sm.wb[i];
+      if (I != I2) tb[(4 * r + q4) * 17 + r16] = d[r];
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (I != I2)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = I2 * 16 + r16, i2 = I * 16 + 4 * r + q4;
+        const double v = tb[r16 * 17 + 4 * r + q4];
+        if (i < k && i2 < k) trans[i + (int64_t)i2 * k] = bad ? nan : v + sm.wb[i];
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
   if (a.wbar)
     for (int i = tid; i < k; i += kThreads) a.wbar[slot * k + i] = bad ? nan : sm.wb[i];
