@@ -9,10 +9,13 @@
 //   solve     W = sqrt(k-1) M^(-1/2), M = C + (k-1)/rho I, and wbar = M^-1 b =
 //             W (W b) / (k-1) (letkf_core.F90:94-210).  An analysis whose
 //             condition bound is above kIsqrtMaxKappa, or that is not finite,
-//             takes the register Jacobi (cold), as do callers that set the
-//             Jacobi's own parameters (k_letkf_plain, k_letkf_wave).  (The
-//             Jacobi from M's Cholesky factor instead of M gave the same
-//             error up to kappa 1e6: that of C and b, not the solver's.)
+//             takes the register Jacobi from M's Cholesky factor L: at these
+//             condition numbers a third to a half fewer sweeps than from M
+//             (2 degrees, every analysis above the limit, k = 48: 10.23 and 6.98
+//             ms a sweep, k = 64: 12.15 and 8.42), the same error up to kappa
+//             1e7 (that of C and b, not the solver's).  Callers that set the
+//             Jacobi's own parameters take it from M (k_letkf_plain,
+//             k_letkf_wave).
 //   out       the transform to HBM, or the ensemble update of the analysis's
 //             column, or of its cube's rows (vertical localisation), fused.
 //
@@ -211,20 +214,32 @@ __device__ __forceinline__ int solve(const dk_batched_args& a, ISmem<KP>& sm, Sy
   }
   Wave<KPJ, DK_GRAM_FP64> w;
   w.patB = true;
+  // from M's Cholesky factor, or from M where a pivot was not positive and finite
+  // (one copy of the loads up to 32 members, where two spill: the core on 4096 analyses
+  // of 16 members 66.8 us, 63.7 so; two above, where the loop spills: 1 degree, k = 64,
+  // 10.05 ms, 10.00 so)
+  bool root = true;
+  constexpr int kCopies = NJ > 2 ? 2 : 1;
+#pragma unroll kCopies
+  for (;;) {
 #pragma unroll
-  for (int J = 0; J < NJJ; ++J)
+    for (int J = 0; J < NJJ; ++J)
 #pragma unroll
-    for (int I = 0; I < NJJ; ++I)
+      for (int I = 0; I < NJJ; ++I)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (I < NJ && J < NJ) w.X[J][I * 4 + r] = elem<NJ>(M, sm.z[0], I, J, r);
-        else w.X[J][I * 4 + r] = 0.0;
-      }
+        for (int r = 0; r < 4; ++r) {
+          if (I < NJ && J < NJ) w.X[J][I * 4 + r] = elem<NJ>(M, sm.z[0], I, J, r);
+          else w.X[J][I * 4 + r] = 0.0;
+        }
+    if (!root) break;
+    root = w.cholesky(k, sm.f, sm.u);
+    if (root) break;
+  }
   __syncthreads();  // z is read before the eigenvectors overwrite it
   bool conv;
   const int sweeps = w.jacobi(a.tol, a.max_sweeps, a.predict != 0, &conv);
   double4_t T[NJJ][NJJ], wb[NJJ];
-  const bool bad = eig_transform<KPJ, DK_GRAM_FP64, false>(w, sm, km1, T, wb);
+  const bool bad = eig_transform<KPJ, DK_GRAM_FP64, false>(w, sm, km1, T, wb, root);
 #pragma unroll
   for (int I = 0; I < NJ; ++I)
 #pragma unroll

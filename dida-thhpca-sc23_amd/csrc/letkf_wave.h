@@ -769,6 +769,54 @@ struct Wave {
     }
   }
 
+  // X, a symmetric positive definite matrix M of order k (rows in pattern B, zero
+  // past k), becomes its lower Cholesky factor L, M = L L^T.  col0, col1: LDS for a
+  // column each.  Returns whether every pivot was positive and finite; otherwise X
+  // is undefined.
+  // Right-looking, a column a step: its four lanes leave it in LDS, every lane takes
+  // its rows and, M being symmetric, its columns of it.  (64 steps of some 600
+  // cycles, half a sweep of the Jacobi.)
+  __device__ __forceinline__ bool cholesky(int k, double* col0, double* col1) {
+    const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+    bool ok = true;
+#pragma unroll
+    for (int J = 0; J < NJ; ++J)
+      for (int cc = 0; cc < 16; ++cc) {
+        const int j = J * 16 + cc;
+        if (j >= k) break;
+        double* v = cc & 1 ? col1 : col0;
+        if (c == cc)
+#pragma unroll
+          for (int I = J; I < NJ; ++I)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[I * 16 + 4 * r + g] = X[J][I * 4 + r];
+        __syncthreads();
+        const double d = v[j];
+        ok &= d > 0.0 && d < __builtin_inf();
+        const double rs = 1.0 / sqrt(d);
+        double lc[NJ];
+#pragma unroll
+        for (int J2 = J; J2 < NJ; ++J2)
+          lc[J2] = J2 * 16 + c > j ? v[J2 * 16 + c] * rs : 0.0;
+#pragma unroll
+        for (int I = J; I < NJ; ++I)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int i = I * 16 + 4 * r + g;
+            const double lr = i >= j ? v[i] * rs : 0.0;
+#pragma unroll
+            for (int J2 = J; J2 < NJ; ++J2)
+              X[J2][I * 4 + r] = J2 == J && c == cc ? lr : fma(-lr, lc[J2], X[J2][I * 4 + r]);
+          }
+      }
+    // above the diagonal, in tiles that no step of their own columns has cleared
+#pragma unroll
+    for (int J = 1; J < NJ; ++J)
+#pragma unroll
+      for (int q = 0; q < J * 4; ++q) X[J][q] = 0.0;
+    return ok;
+  }
+
   // One-sided Jacobi on X.  Returns sweeps; *conv when a sweep rotated
   // nothing, or (predict) when no pair of a sweep had gamma^2 > tol alpha
   // beta, so that the next sweep would rotate nothing.
@@ -987,16 +1035,17 @@ __device__ __forceinline__ void update_rows(int k, int nrow, const double* __res
 
 // W and wbar from the converged columns of w (lambda_j v_j) and b (sm.b):
 // T[I][I2][r] = W(I*16 + 4r + g, I2*16 + c), wb[I][r] = wbar(I*16 + 4r + g).
-// FULLV leaves the eigenvectors in sm.V for the next warm start.  Returns
+// FULLV leaves the eigenvectors in sm.V for the next warm start.  root: the
+// columns are sqrt(lambda_j) v_j, those of a Cholesky factor.  Returns
 // whether a non-finite value was met (T and wb are then not set to NaN yet).
 template <int KP, int GRAM, bool FULLV, class SM>
 __device__ __forceinline__ bool eig_transform(Wave<KP, GRAM>& w, SM& sm, double km1,
                                               double4_t (&T)[KP / 16][KP / 16],
-                                              double4_t (&wb)[KP / 16]) {
+                                              double4_t (&wb)[KP / 16], bool root = false) {
   constexpr int NJ = KP / 16;
   constexpr int LDV = KP + 1;
   const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  // lambda_j = |a_j|; V = A / lambda (to LDS); f = sqrt((k-1)/lambda);
+  // lambda_j = |a_j| (root: |a_j|^2); V = A / |a| (to LDS); f = sqrt((k-1)/lambda);
   // u = V^T b / lambda
   double lam[NJ];
   // a non-finite Yb, d or R^-1 reaches M (then lambda) or b: the analysis is
@@ -1005,7 +1054,8 @@ __device__ __forceinline__ bool eig_transform(Wave<KP, GRAM>& w, SM& sm, double 
   bool bad = false;
 #pragma unroll
   for (int J = 0; J < NJ; ++J) {
-    lam[J] = sqrt(w.colnorm(J));
+    const double n2 = w.colnorm(J);
+    lam[J] = root ? n2 : sqrt(n2);
     bad |= !__builtin_isfinite(lam[J]) || !__builtin_isfinite(sm.b[J * 16 + c]);
   }
   bad = __any(bad);
@@ -1027,13 +1077,14 @@ __device__ __forceinline__ bool eig_transform(Wave<KP, GRAM>& w, SM& sm, double 
   // eigenvector slot J to LDS, with f and u
   auto put_v = [&](int J) {
     const double il = lam[J] > 0.0 ? 1.0 / lam[J] : 0.0;
+    const double ia = root ? sqrt(il) : il;
     double ub = 0.0;
 #pragma unroll
     for (int I = 0; I < NJ; ++I)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int i = row_of(w.patB, I, r, g);
-        const double v = w.X[J][I * 4 + r] * il;
+        const double v = w.X[J][I * 4 + r] * ia;
         sm.V[i + ((FULLV ? J * 16 : 0) + c) * LDV] = v;
         ub += v * sm.b[i];
       }
