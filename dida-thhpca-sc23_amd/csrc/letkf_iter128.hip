@@ -14,8 +14,8 @@
 //   out       W and wbar = M^-1 b = W (W b) / (k-1) to HBM (letkf_core.F90:94-210).
 //
 // An analysis whose condition bound is above kIsqrtMaxKappa, or that is not
-// finite, is marked for the register Jacobi of a second, persistent launch
-// (k_letkf_core_marked; in this kernel its registers and 138 KB of LDS would be
+// finite, is marked for the register Jacobi of a second, persistent launch, from M's
+// Cholesky factor (k_letkf_core_marked; in this kernel its registers and LDS would be
 // everyone's).
 #include <cstring>
 

@@ -325,6 +325,44 @@ struct Jacobi128 {
       __syncthreads();
     }
   }
+  // X (columns J * 32 + gp, rows 8u + sub), a symmetric positive definite matrix M
+  // of order k, zero past k, becomes its lower Cholesky factor: right-looking, a
+  // column a step through LDS (col0, col1 in turn), one barrier each.  Returns whether
+  // every pivot was positive and finite; otherwise X is undefined.
+  __device__ __forceinline__ bool cholesky(int k, int gp, int sub, double* col0, double* col1) {
+    bool ok = true;
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+      for (int cg = 0; cg < 32; ++cg) {
+        const int n = J * 32 + cg;
+        if (n >= k) break;
+        double* v = cg & 1 ? col1 : col0;
+        if (gp == cg)
+#pragma unroll
+          for (int u = 4 * J; u < NR; ++u) v[8 * u + sub] = X[J][u];
+        __syncthreads();
+        const double d = v[n];
+        ok &= d > 0.0 && d < __builtin_inf();
+        const double rs = 1.0 / sqrt(d);
+        double lc[4];
+#pragma unroll
+        for (int J2 = J; J2 < 4; ++J2)
+          lc[J2] = J2 * 32 + gp > n ? v[J2 * 32 + gp] * rs : 0.0;
+#pragma unroll
+        for (int u = 4 * J; u < NR; ++u) {
+          const double lr = 8 * u + sub >= n ? v[8 * u + sub] * rs : 0.0;
+#pragma unroll
+          for (int J2 = J; J2 < 4; ++J2)
+            X[J2][u] = J2 == J && gp == cg ? lr : fma(-lr, lc[J2], X[J2][u]);
+        }
+      }
+    // above the diagonal, in rows that no step of their own columns has cleared
+#pragma unroll
+    for (int J = 1; J < 4; ++J)
+#pragma unroll
+      for (int u = 0; u < 4 * J; ++u) X[J][u] = 0.0;
+    return ok;
+  }
   __device__ __forceinline__ void fold() {
 #pragma unroll
     for (int J = 0; J < 4; ++J) {
@@ -336,9 +374,13 @@ struct Jacobi128 {
   }
 };
 
-template <int LDA, int NTHREADS>
+// CHOL: A is a symmetric positive definite matrix of order k; the sweeps start
+// from its Cholesky factor, and *root tells so (false: a pivot was not positive and
+// finite, and they started from A).  col0, col1: LDS for a column each.
+template <int LDA, int NTHREADS, bool CHOL = false>
 __device__ int jacobi_regs128(double* A, int* flag, double tol, int max_sweeps, bool predict,
-                              bool* converged) {
+                              bool* converged, int k = 0, double* col0 = nullptr,
+                              double* col1 = nullptr, bool* root = nullptr) {
   static_assert(NTHREADS == 256, "32 groups of eight threads");
   static_assert(sizeof(JacobiXbuf) <= sizeof(double) * 128 * LDA, "exchange area fits in A");
   constexpr int NR = Jacobi128::NR;
@@ -356,6 +398,14 @@ __device__ int jacobi_regs128(double* A, int* flag, double tol, int max_sweeps, 
   if (tid == 0) {
     flag[0] = 0;
     flag[2] = 0;
+  }
+  if constexpr (CHOL) {
+    *root = j.cholesky(k, gp, sub, col0, col1);
+    if (!*root)
+#pragma unroll
+      for (int J = 0; J < 4; ++J)
+#pragma unroll
+        for (int u = 0; u < NR; ++u) j.X[J][u] = A[8 * u + sub + j.id[J] * LDA];
   }
   __syncthreads();  // A is read before the exchange area is written
   const double tol2 = tol * tol;

@@ -118,7 +118,7 @@ def test_ill_conditioned_sweep_matches_oracle(cuda, dl, oracle, case):
 
 # The Jacobi in the iteration's kernel runs one wavefront a SIMD above 32 members, that
 # of a caller's jacobi_tol two, from M itself: equal sweeps took 11 to 21 % longer.
-@pytest.mark.parametrize("k", [24, 48, 64])
+@pytest.mark.parametrize("k", [24, 48, 64, 100])
 def test_ill_conditioned_sweeps_start_from_the_cholesky_factor(cuda, dl, k):
     torch = cuda
     cfg, data = _case(dl, k, 1e4)
@@ -128,3 +128,17 @@ def test_ill_conditioned_sweeps_start_from_the_cholesky_factor(cuda, dl, k):
     print(f"  sweeps {st['sweeps_sum']} from L, {st2['sweeps_sum']} from M", flush=True)
     assert st["status"] == 0 and st["max_sweeps_used"] > 4, st
     assert st["sweeps_sum"] < 0.875 * st2["sweeps_sum"]
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("k", [100, 128])
+def test_very_ill_conditioned_sweeps_converge(cuda, dl, k, form):
+    """Condition numbers of 1e7 and more, where cold sweeps of M itself pass the cap."""
+    torch = cuda
+    cfg, data = _case(dl, k, 1e6)
+    print(f"very ill-conditioned k={k} form={form}", flush=True)
+    _, xa, axa, st = _sweep(dl, torch, cfg, data, form=form)
+    print(f"  {st['nonconverged']} of {st['nanal']} not converged, mean sweeps "
+          f"{st['sweeps_sum'] / st['nanal']:.2f}", flush=True)
+    assert st["status"] == 0 and st["nonconverged"] == 0, st
+    assert bool(torch.isfinite(xa).all()) and bool(torch.isfinite(axa).all())
