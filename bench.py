@@ -692,8 +692,9 @@ def main():
         if args.chain_len > 0 and form == dl.FORM_BATCHED:
             extra["chain_len"] = args.chain_len
         if pinned and form == dl.FORM_BATCHED:
-            extra.update(chain_len=int(pinned["chain_len"]),
-                         xcd_tiles=int(pinned.get("xcd_tiles", 0)),
+            if gram != dl.GRAM_FP64 or cfg.k <= 64:  # (no chains: a length asks for the Jacobi's)
+                extra["chain_len"] = int(pinned["chain_len"])
+            extra.update(xcd_tiles=int(pinned.get("xcd_tiles", 0)),
                          bin_deg=float(pinned.get("bin_deg", 0.0)))
             if pinned.get("bucketed"):
                 extra["bucket_chain"] = [int(b) for b in pinned["bucket_chain"]]

@@ -1423,7 +1423,6 @@ int dida_letkf_autotune(dida_letkf_ctx *c, const dida_letkf_obs *o, const double
     const int32_t chains[6] = {2, 4, 8, 16, 32, 64};
     const double bd1 = best_bd;
     const int chains_used = batched && !c->iter;
-    if (c->iter) best_cl = chains[2]; /* no chains: every length is the same */
     for (int ic = 0; ic < 6 && chains_used && !rc; ++ic)
         for (int it = 0; it < 2 && !rc; ++it)
             if (!(bd1 == best_bd && chains[ic] == best_cl && it == best_tl && !best_bk))
@@ -1472,7 +1471,9 @@ int dida_letkf_autotune(dida_letkf_ctx *c, const dida_letkf_obs *o, const double
     if (rc) return rc;
     rc = dida_letkf_sweep(c, o, xb, axb, xa, axa, stream);
     if (rc < 0) return rc;
-    out->chain_len = batched ? c->chain_len : 0;
+    /* (0 where the context iterates above 64 members: a length there asks for the
+     * chains of the Jacobi) */
+    out->chain_len = batched && !(c->iter && c->prm.nanals > 64) ? c->chain_len : 0;
     out->bin_deg = c->bin_deg;
     out->ms_best = best_ms;
     out->xcd_tiles = batched ? c->ngroup > 0 : 0;

@@ -295,7 +295,9 @@ int dida_letkf_graph_launch(dida_letkf_ctx *ctx, void *stream);
  * timed twice (HIP events, minimum); xa/axa hold the result of a sweep with
  * the kept layout on return.  Synchronises. */
 typedef struct dida_letkf_tuning {
-    int32_t chain_len;          /* kept (batched form; 0 for the plain form) */
+    int32_t chain_len;          /* kept (batched form; 0 for the plain form, and above 64
+                                   members for FP64 contexts that iterate, which have no
+                                   chains and which a length would turn to the Jacobi) */
     int32_t ncand;              /* layouts timed */
     double bin_deg;             /* kept */
     double ms_initial;          /* sweep time with the layout on entry and the kept
