@@ -113,6 +113,12 @@ __device__ __forceinline__ void store4(float* p, const double4_t& v, int n) {
   }
 }
 
+// What is taken from the members' deviations: their mean; a row whose xbar_b is not
+// finite has no finite member, as where xbar_b is added before the mean is taken.
+__device__ __forceinline__ double centre_of(double mean, double xbar) {
+  return __builtin_isfinite(xbar) ? mean : __builtin_nan("");
+}
+
 template <int KP>
 __global__ __launch_bounds__(64, KP <= 32 ? 4 : KP == 48 ? 2 : 1) void k_update_cols(dk_update_args u,
                                                                       dk_update_grid gr) {
@@ -204,8 +210,9 @@ __global__ __launch_bounds__(64, KP <= 32 ? 4 : KP == 48 ? 2 : 1) void k_update_
 #pragma unroll
       for (int E = 1; E < NJ; ++E) s4 += D[E];
       const double mean = sum_g((s4[0] + s4[1]) + (s4[2] + s4[3])) / (double)k;
+      const double centre = centre_of(mean, xbar);
 #pragma unroll
-      for (int E = 0; E < NJ; ++E) D[E] -= mean;
+      for (int E = 0; E < NJ; ++E) D[E] -= centre;
       double fac = 1.0;
       if (u.rtps) {
         double4_t q4 = zero;
@@ -361,8 +368,9 @@ __global__ __launch_bounds__(256, 2) void k_update_cols128(dk_update_args u,
       __syncthreads();
       const double mean =
           ((sv[buf][0][c] + sv[buf][1][c]) + (sv[buf][2][c] + sv[buf][3][c])) / (double)k;
-      D[0] -= mean;
-      D[1] -= mean;
+      const double centre = centre_of(mean, xbar);
+      D[0] -= centre;
+      D[1] -= centre;
       if (u.rtps) {
         double q = 0.0;
 #pragma unroll
