@@ -291,9 +291,9 @@ struct Part {
     publish(T2, z1);
     const double kap = kappa(T2, z1, a0, sm);
     // (a0 outside this range could lose M^2 to underflow)
-    if (!(kap <= kIsqrtMaxKappa && a0 > 1e-100 && a0 < 1e100)) {
-      return 0;
-    }
+    // (the same in every thread, and scalar: barriers follow)
+    const bool steps_ok = kap <= kIsqrtMaxKappa && a0 > 1e-100 && a0 < 1e100;
+    if (!__builtin_amdgcn_readfirstlane(steps_ok)) return 0;
     int cls = 0;
 #pragma unroll
     for (int i = 0; i < kIsqrtPlans - 1; ++i) cls += kap > kIsqrtPlan[i].kappa;
@@ -381,7 +381,9 @@ __global__ __launch_bounds__(256) void k_letkf_iter128(dk_core_args a) {
   const int o = b / 64 * 64 + b % 8 * 8 + b / 8 % 8;
   if (o >= a.nanal) return;
   const int aid = a.aid0 + o;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  // (scalar: the barriers of the wavefronts' parts stand in branches that it decides)
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int k = a.k;
   PhaseClock clk(a.phase_clk);
   const int64_t off = a.offset ? a.offset[aid] - a.base : aid * (int64_t)a.max_p;
