@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import sys
 from dataclasses import dataclass
 
 import numpy as np
@@ -429,10 +430,11 @@ def letkf_core(hxens: np.ndarray, rdiaginv, dep, rloc, inflation: float, pflag: 
 
 def _by_rows(trans, batch, k):
     """(batch, i, j) arrays of the library's trans(i, j) at i + j k; large ones by
-    torch, which transposes on all host threads."""
-    if trans.size < 1 << 16:
+    torch, which transposes on all host threads, in a program that has loaded it (the
+    import alone takes longer than numpy's transpose)."""
+    torch = sys.modules.get("torch")
+    if torch is None or trans.size < 1 << 16:
         return trans.reshape(batch, k, k).transpose(0, 2, 1).copy()
-    import torch
     return torch.from_numpy(trans).view(batch, k, k).transpose(1, 2).contiguous().numpy()
 
 
