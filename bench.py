@@ -140,22 +140,28 @@ def selection_bytes(k, nobs, nobsl_sum):
     return nobs * (8.0 * k + 32.0) + 12.0 * nobsl_sum
 
 
-def kernel_roofline(cfg, st, head, kernel_ms, config, scale, layout=None):
-    """Roofline of the dominant kernel (the batched form's fused kernel, or
-    the plain form's transform kernel) from algorithmic flops per sweep:
-    Gram 2k^2 p (three half-precision MFMA passes in the split-x3 forms),
-    b 2kp, eigensolve 9k^3 + W 2k^3 + wbar 4k^2 per analysis (nominal), and,
-    when fused, the update 2k^2 n + 2kn.  The peak is the rate at which the
+def kernel_roofline(cfg, st, head, kernel_ms, config, scale, layout=None, chain_len=0,
+                    state_f32=False):
+    """Roofline of the dominant kernel (the one of the transform stage) from
+    algorithmic flops per sweep: Gram 2k^2 p (three half-precision MFMA passes
+    in the split-x3 forms), b 2kp, per analysis the solve (FP64 forms: twelve
+    symmetric products of k^3 flops, the usual number, and wbar 4k^2; the
+    Jacobi of the others, and of FP64 forms above 64 members with a chain
+    length: eigensolve 9k^3 + W 2k^3 + wbar 4k^2, nominal), and, when fused,
+    the update 2k^2 n + 2kn.  The peak is the rate at which the
     mix would run with each part at its own published peak (BF16/FP16 dense
     MFMA 2.5 PFLOP/s, FP64 78.6 TFLOP/s), so frac = (time at peak) / time."""
     k, n, ncol = cfg.k, 1 + 3 * cfg.nz, cfg.nlat * cfg.nlon
     p_sum = float(st["nobsl_sum"])
     gram = 2.0 * k * k * p_sum
-    fp64 = 2.0 * k * p_sum + ncol * (11.0 * k ** 3 + 4.0 * k * k)
-    fused = head != "plain_fp64" and k <= 64   # k > 64: chained analyses, update apart
+    all64 = head.endswith("fp64")
+    iterates = all64 and not (k > 64 and chain_len > 0)
+    # up to 64 members the update is fused, but for the plain form's FP32 state
+    fused = k <= 64 and not (head == "plain_fp64" and state_f32)
+    fp64 = 2.0 * k * p_sum + ncol * ((12.0 if iterates else 11.0) * k ** 3 + 4.0 * k * k)
     if fused:
         fp64 += ncol * (2.0 * k * k * n + 2.0 * k * n)
-    if head.endswith("fp64"):
+    if all64:
         half, fp64 = 0.0, fp64 + gram
     else:
         half = (3.0 if head.endswith("x3") else 1.0) * gram
@@ -167,18 +173,24 @@ def kernel_roofline(cfg, st, head, kernel_ms, config, scale, layout=None):
     # 4k + 24 with the FP32 rows of the split half-precision Grams; mostly
     # served from L2, neighbouring columns share obs) and, fused, the update's
     # 2kn f64 + 2n f64 per column
-    row_bytes = 8.0 if head.endswith("fp64") or not fused else 4.0
-    gathered = p_sum * (row_bytes * k + 24.0)
+    gathered = p_sum * ((8.0 if all64 else 4.0) * k + 24.0)
     upd = ncol * (2.0 * k * n * 8 + 2.0 * n * 8) if fused else 0.0
     traffic = measured_traffic(head, config, scale, layout)
+    if iterates:
+        kernel = "k_letkf_iter (Gram, iteration, transform" if k <= 64 else \
+            "k_letkf_iter128 (Gram, iteration, transform"
+        kernel += ", update)" if fused else ")"
+    elif k <= 64:
+        kernel = "k_letkf_wave (fused Gram, eigensolve, transform, update)"
+    elif head != "plain_fp64":
+        kernel = "k_letkf_chain_f64 (chained Gram, warm-started eigensolve, transform)"
+    else:
+        kernel = "k_letkf_core_f64 (Gram, eigensolve, transform)"
     return {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
             "frac": achieved / peak if achieved else None, "traffic": traffic,
             "traffic_key": traffic_key(head, config, scale, layout) if layout else None,
-            "kernel": "k_letkf_wave (fused Gram, eigensolve, transform, update)" if fused
-            else ("k_letkf_chain_f64 (chained Gram, warm-started eigensolve, transform)"
-                  if head != "plain_fp64" else "k_letkf_core_f64 (Gram, eigensolve, transform)"),
-            "kernel_ms": kernel_ms, "flops_per_launch": flops, "half_flops": half,
-            "fp64_flops": fp64,
+            "kernel": kernel, "kernel_ms": kernel_ms, "flops_per_launch": flops,
+            "half_flops": half, "fp64_flops": fp64,
             "algorithmic_bytes": {"obs_gathered": gathered, "update": upd},
             "hbm_frac_algorithmic": (gathered + upd) / (kernel_ms / 1e3) / (HBM_PEAK_GBS * 1e9)
             if kernel_ms > 0 else None}
@@ -752,7 +764,8 @@ def main():
         layout = {"chain_len": args.chain_len or (32 if cfg.k > 64 else 8),
                   "xcd_tiles": 0}   # library defaults
     roofline = kernel_roofline(cfg, st, head, r["stages"]["transform"], args.config,
-                               args.scale, layout)
+                               args.scale, layout, forms[head][2].get("chain_len", 0),
+                               args.state_f32)
 
     out_forms = {}
     for name, rr in res.items():
