@@ -254,8 +254,9 @@ __global__ __launch_bounds__(64, KP <= 32 ? 4 : KP == 48 ? 2 : 1) void k_update_
 // Xa' are stored in; all arithmetic is FP64.  Measured
 // at 1 degree, k = 128, FP32 state, 97 rows (15 GB, 0.2 TFLOP): 9.9 ms with rows
 // staged in LDS a tile at a time, nothing in flight behind, 8.1 ms with whole rows
-// in flight, 5.6 ms so; a tile a wavefront, eight wavefronts: 6.7 ms (168
-// registers, one workgroup a CU) and 11.5 ms (128, spilling).
+// in flight, 5.6 ms so (at NT = 8 the bound of 256 spills 39 registers, 44 with FP64
+// state; at 7, 3); a tile a wavefront, eight wavefronts: 6.7 ms (168 registers, one
+// workgroup a CU) and 11.5 ms (128, spilling more).
 template <int NT, typename S>
 __global__ __launch_bounds__(256, 2) void k_update_cols128(dk_update_args u,
                                                                dk_update_grid gr) {

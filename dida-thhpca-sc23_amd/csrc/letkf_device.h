@@ -183,11 +183,11 @@ struct H16<DK_GRAM_FP16X3> {
 template <>
 struct H16<DK_GRAM_BF16> : H16<DK_GRAM_BF16X3> {};
 
-// Per-phase clock accounting (wall_clock64), one thread per workgroup.
 // The bits (a NaN no computation returns) that k_letkf_iter128 leaves in the first
 // value of a transform to be computed by the Jacobi.
 constexpr long long kMarkBits = 0x7FF8D1DA00000001LL;
 
+// Per-phase clock accounting (wall_clock64), one thread per workgroup.
 struct PhaseClock {
   unsigned long long* out;
   unsigned long long t;

@@ -1799,6 +1799,14 @@ int dida_letkf_core_batch_dev_noalloc(int32_t batch, int32_t max_obs, int32_t na
  * synchronisation (k = 20, 245 obs: 131 -> 48 us).  Larger ones: a few
  * threads, each with two pinned slots, pack (and for REAL(4) widen) one slot
  * while the other travels (512 analyses, k = 64, up to 2100 obs: 23.8 -> 11.2 ms).
+ * On either side of the values, the same 512 analyses (64 of them, 300 of k = 24, 300
+ * obs): 1, 2, 4 and 8 threads 14.7, 11.7, 11.7, 11.9 ms (2.13, 1.89, 1.88, 2.00; 0.57,
+ * 0.59, 0.61, 0.61); slots of 1, 2, 4, 8 and 16 MiB 17.3, 13.3, 11.7, 11.1, 11.2 ms (2.48,
+ * 2.01, 1.92, 1.92, 2.07; 0.74, 0.64, 0.61, 0.76, 0.93).  Small calls end at 32 KiB, 256
+ * KiB, 1 MiB: one analysis of k = 20, 245 obs 65, 43, 43 us, k = 64, 900 obs 180, 179,
+ * 143 us, 30 of k = 20, 245 obs 124, 124, 124 us (8 MiB: 85): above 256 KiB the caller's
+ * thread alone would pack up to 40 % faster than the threads, whose start and events
+ * cost some 35 us.
  *
  * Buffers are kept per calling thread, and freed when it ends: the arena of
  * the largest call, the two small pinned buffers, and the slots (DIDA_SLOTS of

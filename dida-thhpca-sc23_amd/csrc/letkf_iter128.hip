@@ -10,7 +10,10 @@
 //             KB at NT = 8), an element above the diagonal from the transposed
 //             tile: a wavefront reads at most 10 operands for 9 MFMAs of 64
 //             cycles, 160 of 576 LDS cycles, so the matrix units are the bound
-//             (288 MFMAs a wavefront and product at NT = 8).
+//             (288 MFMAs a wavefront and product at NT = 8).  T, T^2, P and Z and the
+//             operands of two steps fit 512 registers up to NT = 7; at NT = 8 323
+//             spill (batched sweep of 80 x 160 columns, k = 112 and 113: 7.0 and 10.0
+//             ms, 1.43 times for 1.47 times the MFMAs).
 //   out       W and wbar = M^-1 b = W (W b) / (k-1) to HBM (letkf_core.F90:94-210).
 //
 // An analysis whose condition bound is above kIsqrtMaxKappa, or that is not

@@ -23,7 +23,7 @@
 // step; the level weight (two logarithms a member, one of the obs pressure
 // and a division) serves every variable.  100 000 single-level records of
 // u, v, T at 1 degree, 32 levels, k = 64: 808 -> 491 us; what is left is the
-// gather of random 512-byte rows (1.6 GB fetched, 3.5 TB/s; 908 VALU
+// gather of random 512-byte rows (1.6 GB fetched, 3.3 TB/s; 908 VALU
 // instructions a record).
 #include "letkf_device.h"
 #include "letkf_kernels.h"

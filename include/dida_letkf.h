@@ -79,7 +79,9 @@ typedef struct dida_letkf_params {
     int32_t chain_len;          /* batched form: adjacent columns per work item,
                                    each warm-starting the next one's eigensolve
                                    (0: automatic; see jacobi_max_sweeps) */
-    int32_t warm_start;         /* batched form: 1 to warm-start along chains */
+    int32_t warm_start;         /* batched form: 1 to warm-start along chains (without
+                                   chains, as FP64 analyses that iterate, it has no
+                                   effect; nor have xcd_tiles and bucket_chain) */
     int32_t jacobi_predict;     /* 1 ends the eigensolve after a sweep whose largest
                                    |a_p.a_q|^2 / (|a_p|^2 |a_q|^2) is <= tol (the
                                    next sweep would rotate nothing if convergence
@@ -198,11 +200,10 @@ void letkf_core_batch_r4_(const int32_t *batch, const int32_t *batch_large_matri
 
 /* Status-returning batched core on device pointers (same layout as
  * letkf_core_batch_), enqueued on `stream` (a hipStream_t, NULL = default).
- * info[batch] (optional) receives the solver's count (k <= 64: the steps of
- * its polynomial iteration, or the Jacobi sweeps of an analysis whose
- * condition number is above the iteration's limit; above: Jacobi sweeps), -1
- * when the eigensolve hit the sweep cap, or -2 when M or b was not finite
- * (trans and overline_w are then NaN). */
+ * info[batch] (optional) receives the solver's count (the steps of its polynomial
+ * iteration, 2 to 4, or the Jacobi sweeps of an analysis whose condition bound is
+ * above the iteration's limit), -1 when the eigensolve hit the sweep cap, or -2
+ * when M or b was not finite (trans and overline_w are then NaN). */
 int dida_letkf_core_batch_dev(int32_t batch, int32_t max_obs, int32_t nanals,
                               const int32_t *nobsl, const double *hxens, const float *rdiaginv,
                               const double *dep, const double *rloc, double *trans,
